@@ -7,22 +7,9 @@
 // Writing b for the bit a butterfly pairs (b = log N - 1 - s forward), both
 // directions read twiddle (N + j) >> (b + 1) for the lower element j.
 //
-// Two kernel families. Here: one workgroup transforms one limb-polynomial
-// on chip (N <= 16384). In ntt_split.hip: a column pass plus a row pass of
-// single-wavefront workgroups (N >= 8192). The whole-polynomial kernel moves
-// each coefficient through HBM once but, at N = 16384, fills a CU's LDS, so
-// a CU cannot overlap one polynomial's loads with another's arithmetic; the
-// split kernels move the data twice but keep many wavefronts per CU. The
-// whole-polynomial kernel's time grows in steps of one round of workgroups
-// (one per CU) and a round takes a transform's time however few workgroups
-// it holds, while the split kernels spread every transform over 16
-// workgroups. Measured on MI355X at N = 16384 (forward, 4-limb chain): 4
-// transforms 23.8 us whole against 11.0 us split, 64: 25.2 against 19.5,
-// 128: 26.5 against 32.6, 256: 29.2 against 35.9; from 384 transforms on the
-// split kernels win again (1792: 197 us against 256 us). So batches of
-// NTT_WHOLE_MIN_JOBS = 96 to NTT_WHOLE_MAX_JOBS = 256 (the CU count) use the
-// first, the others the second (the segment-sum epilogue exists in the first
-// only).
+// One workgroup transforms one limb-polynomial on chip (N <= 16384); the split
+// kernels (ntt_split.hip) serve the other sizes and batches (ntt_launch.hip).
+// The kernels are templates of the chain's arithmetic above 2^41 (BIG).
 //
 // Whole-polynomial kernel: T = N/16 threads hold 16 coefficients each in
 // registers; a register pass performs up to 4 butterfly stages on the
@@ -42,21 +29,9 @@
 // LDS wait counter and hold up every exchange. The fused load/store
 // operations are template parameters, so each kernel carries only its own.
 #include "ntt_arith.h"
+#include "ntt_kernels.h"
 
 namespace th {
-
-constexpr int NTT_WHOLE_MAX_LOGN = 14;
-#ifndef NTT_WHOLE_MAX_JOBS
-#define NTT_WHOLE_MAX_JOBS 256
-#endif
-#ifndef NTT_WHOLE_MIN_JOBS
-#define NTT_WHOLE_MIN_JOBS 96
-#endif
-hipError_t launch_ntt_split(int logn, bool inverse, const NttArgs& a, uint32_t njobs, hipStream_t s);
-hipError_t launch_rescale_split(int logn, const NttArgs& inv, uint32_t ninv, const NttArgs& fwd, uint32_t nf,
-                                hipStream_t s);
-hipError_t launch_encrypt_split(int logn, const NttArgs& a, uint32_t ninputs, uint32_t L, uint32_t limb_mask,
-                                const EncDot& dot, const uint64_t* pkp, uint64_t* cts, hipStream_t s);
 
 template <int LOGN>
 struct Shape {
@@ -113,6 +88,8 @@ __device__ __forceinline__ uint32_t jhi_of(uint32_t tid) {
 
 // ------------------------------------------------------------------ register passes
 // Forward stages for bits BHI down to BLO on the layout with register bits [LO, LO+LE).
+// The first pass (BHI = LOGN - 1) works on values as loaded and folds nothing
+// (PmArith).
 template <int LOGN, int LO, int BHI, int BLO, class A>
 __device__ __forceinline__ void fwd_pass(typename A::V (&x)[Shape<LOGN>::E], uint32_t tid,
                                          GPtr<typename A::Tw> tw, const A& ar) {
@@ -127,7 +104,7 @@ __device__ __forceinline__ void fwd_pass(typename A::V (&x)[Shape<LOGN>::E], uin
       if (k & (1 << rb)) continue;
       const int k2 = k | (1 << rb);
       const typename A::Tw t = ld16(tw, base | (uint32_t)(k >> (rb + 1)));
-      ar.fwd(x[k], x[k2], t);
+      ar.fwd(x[k], x[k2], t, BHI != LOGN - 1 && b == BHI);
     }
   }
 }
@@ -138,6 +115,7 @@ __device__ __forceinline__ void inv_pass(typename A::V (&x)[Shape<LOGN>::E], uin
                                          GPtr<typename A::Tw> tw, const A& ar, const LimbConst& lc) {
   using S = Shape<LOGN>;
   const uint32_t jhi = jhi_of<LOGN, LO>(tid);
+  constexpr InvPlan<BLO - LO, BHI - BLO + 1> plan;
 #pragma unroll
   for (int b = BLO; b <= BHI; ++b) {
     const int rb = b - LO;
@@ -158,7 +136,8 @@ __device__ __forceinline__ void inv_pass(typename A::V (&x)[Shape<LOGN>::E], uin
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int k = 0; k < S::E; ++k)
-        if (!(k & (1 << rb))) ar.inv(x[k], x[k | (1 << rb)], t[k >> (rb + 1)]);
+        if (!(k & (1 << rb)))
+          ar.inv(x[k], x[k | (1 << rb)], t[k >> (rb + 1)], plan.small[b - BLO][k], plan.fold[b - BLO][k]);
     }
   }
   if (BHI != LOGN - 1) {
@@ -231,13 +210,13 @@ __device__ __forceinline__ void inv_passes(typename A::V (&x)[Shape<LOGN>::E], t
 // with the rescale constants *rc (the coefficient-domain end of a rescaled
 // decryption, rescale_decrypt_kernel).
 template <int LOGN, int END, bool RESCALED, class A>
-__device__ __forceinline__ void segsum_store(const typename A::V (&x)[Shape<LOGN>::E], const A& ar, uint64_t q,
-                                             uint32_t tid, const double* segw, uint32_t cols, double* seg,
+__device__ __forceinline__ void segsum_store(const typename A::V (&x)[Shape<LOGN>::E], const A& ar,
+                                             const LimbConst& lc, uint32_t tid, const double* segw, uint32_t cols, double* seg,
                                              double scale, const uint64_t* xl, const RescaleConst* rcp,
                                              void* lds_raw) {
   using S = Shape<LOGN>;
   constexpr int MAXC = NTT_SEGSUM_FUSED_MAX_COLS;
-  const uint64_t half = q >> 1;
+  const uint64_t q = lc.q, half = q >> 1;
   using D2 = double __attribute__((ext_vector_type(2)));
   const GPtr<D2> W = gld(reinterpret_cast<const D2*>(segw));
   double acc[MAXC];
@@ -262,8 +241,8 @@ __device__ __forceinline__ void segsum_store(const typename A::V (&x)[Shape<LOGN
     if constexpr (RESCALED) {
       const uint64_t xv = xq[k % PF];
       if (k + PF < S::E) xq[k % PF] = gld(xl)[elem<S::LE, END>(tid, k + PF)];
-      const uint64_t xr = xv < rc.q ? xv : mulmod_barrett(xv, 1, rc.b);
-      m = csub(shoup_lazy(submod(m, xr, q), rc.inv, rc.inv_s, q), q);
+      const bool whole = std::is_same_v<A, PmArith> || xv < rc.q;
+      m = rescaled_coefficient<A>(m, whole ? xv : mulmod_barrett(xv, 1, rc.b), rc, lc);
     }
     const double v = m > half ? -(double)(q - m) : (double)m;
     const D2 p = wq[k % PF];  // W_0[j], 2 cos(2 phi_j) at j = elem(tid, k)
@@ -307,7 +286,7 @@ __device__ __forceinline__ void run_ntt(const uint64_t* __restrict__ src, uint64
   typename A::V* lds = reinterpret_cast<typename A::V*>(lds_raw);
   if constexpr (!INV) {
 #pragma unroll
-    for (int k = 0; k < S::E; ++k) x[k] = ar.load(op(src, elem<S::LE, S::COAL_LO>(tid, k)));
+    for (int k = 0; k < S::E; ++k) x[k] = ar.load(op.template at<A>(src, elem<S::LE, S::COAL_LO>(tid, k)));
     const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd));
     fwd_passes<LOGN, LOGN, S::COAL_LO, A>(x, lds, tid, tw, ar);
 #pragma unroll
@@ -318,11 +297,11 @@ __device__ __forceinline__ void run_ntt(const uint64_t* __restrict__ src, uint64
   } else {
     const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.inv));
 #pragma unroll
-    for (int k = 0; k < S::E; ++k) x[k] = ar.load(op(src, elem<S::LE, S::WAVE_LO>(tid, k)));
+    for (int k = 0; k < S::E; ++k) x[k] = ar.load(op.template at<A>(src, elem<S::LE, S::WAVE_LO>(tid, k)));
     inv_passes<LOGN, 0, S::WAVE_LO, A>(x, lds, tid, tw, ar, lc);
     constexpr int END = inv_end_lo<LOGN>();
     if constexpr (SOp::kind == NTT_STORE_SEGSUM) {
-      segsum_store<LOGN, END, false>(x, ar, lc.q, tid, so.segw, so.cols, so.seg, so.scale, nullptr, nullptr, lds_raw);
+      segsum_store<LOGN, END, false>(x, ar, lc, tid, so.segw, so.cols, so.seg, so.scale, nullptr, nullptr, lds_raw);
     } else {
 #pragma unroll
       for (int k = 0; k < S::E; ++k) gdst[elem<S::LE, END>(tid, k)] = ar.inv_store(x[k]);
@@ -330,7 +309,7 @@ __device__ __forceinline__ void run_ntt(const uint64_t* __restrict__ src, uint64
   }
 }
 
-template <int LOGN, bool INV, uint32_t LD, uint32_t ST>
+template <class BIG, int LOGN, bool INV, uint32_t LD, uint32_t ST>
 __global__ __launch_bounds__(Shape<LOGN>::T) void ntt_kernel(NttArgs a) {
   extern __shared__ uint64_t lds[];
   const uint32_t job = blockIdx.x;
@@ -351,10 +330,7 @@ __global__ __launch_bounds__(Shape<LOGN>::T) void ntt_kernel(NttArgs a) {
     limb = a.limb_base + job % a.limb_mod;
   }
   const LimbConst& lc = a.lc[limb];
-  if (lc.fp64)
-    run_ntt<LOGN, INV, Fp64Arith>(src, dst, lc, op, so, lds);
-  else
-    run_ntt<LOGN, INV, IntArith>(src, dst, lc, op, so, lds);
+  with_arith<BIG>(lc, [&]<class A>() { run_ntt<LOGN, INV, A>(src, dst, lc, op, so, lds); });
 }
 
 // One rescaled product's decryption on limb 0, with its segment sums
@@ -387,123 +363,72 @@ __device__ __forceinline__ void run_rescale_decrypt(const RescaleDecryptArgs& a,
 #pragma unroll
     for (int k = 0; k < S::E; ++k) {
       const uint64_t v = y[elem<S::LE, S::COAL_LO>(tid, k)];
-      x[k] = ar.load(v < q ? v : mulmod_barrett(v, 1, rcp->b));
+      x[k] = ar.load(std::is_same_v<A, PmArith> || v < q ? v : mulmod_barrett(v, 1, rcp->b));  // pm: below 3q
     }
   }
   fwd_passes<LOGN, LOGN, S::COAL_LO, A>(x, lds, tid, gld(reinterpret_cast<const typename A::Tw*>(lc.fwd)), ar);
   {
-    // D pt - NTT(r_1) s: Montgomery products with pt and s in Montgomery
-    // form, each in [0, 2q), so the difference plus 2q is in (0, 4q): the
-    // integer inverse's input range; the FP64 inverse gets it canonical
+    // D pt - NTT(r_1) s, pt and s prepared
     const GPtr<uint64_t> d = gld(jb.d), p = gld(jb.ptm), sk = gld(a.skm);
-    const uint64_t q = lc.q, two_q = 2 * lc.q;
 #pragma unroll
     for (int k = 0; k < S::E; ++k) {
       const uint32_t i = elem<S::LE, S::WAVE_LO>(tid, k);
-      const uint64_t u = mont_mul(d[i], p[i], bc);
-      const uint64_t t = mont_mul(ar.fwd_store(x[k]), sk[i], bc);
-      uint64_t e = u + two_q - t;
-      if constexpr (std::is_same_v<A, Fp64Arith>) e = csub(csub(e, two_q), q);
-      x[k] = ar.load(e);
+      x[k] = ar.load(prepared_difference(ar, d[i], p[i], x[k], sk[i], bc));
     }
   }
   inv_passes<LOGN, 0, S::WAVE_LO, A>(x, lds, tid, gld(reinterpret_cast<const typename A::Tw*>(lc.inv)), ar, lc);
-  segsum_store<LOGN, inv_end_lo<LOGN>(), true>(x, ar, lc.q, tid, a.segw, a.cols, jb.seg, jb.scale, jb.x, rcp,
+  segsum_store<LOGN, inv_end_lo<LOGN>(), true>(x, ar, lc, tid, a.segw, a.cols, jb.seg, jb.scale, jb.x, rcp,
                                                lds_raw);
 }
 
-template <int LOGN>
+template <class BIG, int LOGN>
 __global__ __launch_bounds__(Shape<LOGN>::T) void rescale_decrypt_kernel(RescaleDecryptArgs a) {
   extern __shared__ uint64_t lds[];
   const RescaleDecryptJob jb = a.jobs[blockIdx.x];
   const LimbConst& lc = a.lc[0];
-  if (lc.fp64)
-    run_rescale_decrypt<LOGN, Fp64Arith>(a, jb, lc, lds);
-  else
-    run_rescale_decrypt<LOGN, IntArith>(a, jb, lc, lds);
+  with_arith<BIG>(lc, [&]<class A>() { run_rescale_decrypt<LOGN, A>(a, jb, lc, lds); });
 }
 
-template <int LOGN>
+template <class BIG, int LOGN>
 static hipError_t launch_rescale_decrypt_t(const RescaleDecryptArgs& a, uint32_t njobs, hipStream_t s) {
-  const hipError_t e = allow_full_lds<rescale_decrypt_kernel<LOGN>>();
+  const hipError_t e = allow_full_lds<rescale_decrypt_kernel<BIG, LOGN>>();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((rescale_decrypt_kernel<LOGN>), dim3(njobs), dim3(Shape<LOGN>::T),
+  hipLaunchKernelGGL((rescale_decrypt_kernel<BIG, LOGN>), dim3(njobs), dim3(Shape<LOGN>::T),
                      (size_t)Shape<LOGN>::LDS_ELEMS * 8, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_rescale_decrypt(int logn, const RescaleDecryptArgs& a, uint32_t njobs, hipStream_t s) {
+template <class BIG>
+hipError_t launch_rescale_decrypt_whole(int logn, const RescaleDecryptArgs& a, uint32_t njobs, hipStream_t s) {
   if (njobs == 0) return hipSuccess;
   if (a.cols < 1 || a.cols > NTT_SEGSUM_FUSED_MAX_COLS) return hipErrorInvalidValue;
   switch (logn) {
-    case 10: return launch_rescale_decrypt_t<10>(a, njobs, s);
-    case 11: return launch_rescale_decrypt_t<11>(a, njobs, s);
-    case 12: return launch_rescale_decrypt_t<12>(a, njobs, s);
-    case 13: return launch_rescale_decrypt_t<13>(a, njobs, s);
-    case 14: return launch_rescale_decrypt_t<14>(a, njobs, s);
+    case 10: return launch_rescale_decrypt_t<BIG, 10>(a, njobs, s);
+    case 11: return launch_rescale_decrypt_t<BIG, 11>(a, njobs, s);
+    case 12: return launch_rescale_decrypt_t<BIG, 12>(a, njobs, s);
+    case 13: return launch_rescale_decrypt_t<BIG, 13>(a, njobs, s);
+    case 14: return launch_rescale_decrypt_t<BIG, 14>(a, njobs, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-template <int LOGN, bool INV>
+template <class BIG, int LOGN, bool INV>
 static hipError_t launch_one(const NttArgs& a, uint32_t njobs, hipStream_t s) {
   using S = Shape<LOGN>;
   const size_t lds = (size_t)S::LDS_ELEMS * 8;
   return with_ops<INV>(a.jobs ? a.load : NTT_LOAD_NONE, a.jobs ? a.store : NTT_STORE_NONE,
                   [&]<uint32_t LD, uint32_t ST>() -> hipError_t {
-                    const hipError_t e = allow_full_lds<ntt_kernel<LOGN, INV, LD, ST>>();
+                    const hipError_t e = allow_full_lds<ntt_kernel<BIG, LOGN, INV, LD, ST>>();
                     if (e != hipSuccess) return e;
-                    hipLaunchKernelGGL((ntt_kernel<LOGN, INV, LD, ST>), dim3(njobs), dim3(S::T), lds, s, a);
+                    hipLaunchKernelGGL((ntt_kernel<BIG, LOGN, INV, LD, ST>), dim3(njobs), dim3(S::T), lds, s, a);
                     return hipGetLastError();
                   });
 }
 
-// Sizes and batches the whole-polynomial kernel cannot serve.
-static bool whole_unavailable(int logn, uint32_t njobs) {
-  return logn >= NTT_SPLIT_MIN_LOGN && (logn > NTT_WHOLE_MAX_LOGN || njobs > NTT_WHOLE_MAX_JOBS);
-}
-static bool use_split(int logn, uint32_t njobs) {
-  return whole_unavailable(logn, njobs) || (logn >= NTT_SPLIT_MIN_LOGN && njobs < NTT_WHOLE_MIN_JOBS);
-}
-
-hipError_t launch_rescale(int logn, const NttArgs& inv, uint32_t ninv, const NttArgs& fwd, uint32_t nfwd,
-                          hipStream_t s) {
-  if (ninv == 0) return hipSuccess;
-  if (use_split(logn, nfwd) && inv.jobs && fwd.jobs && nfwd % ninv == 0 && inv.store == NTT_STORE_NONE &&
-      fwd.load == NTT_LOAD_REDUCE)
-    return launch_rescale_split(logn, inv, ninv, fwd, nfwd / ninv, s);
-  hipError_t e = launch_ntt(logn, true, inv, ninv, s);
-  if (e != hipSuccess) return e;
-  return launch_ntt(logn, false, fwd, nfwd, s);
-}
-
-bool encrypt_limbs_supported(int logn) { return logn >= NTT_SPLIT_MIN_LOGN && logn <= NTT_MAX_LOGN; }
-
-hipError_t launch_encrypt(int logn, const NttArgs& a, uint32_t ninputs, uint32_t L, uint32_t limb_mask,
-                          const EncDot& dot, const uint64_t* pkp, uint64_t* cts, bool* combined, hipStream_t s) {
-  *combined = false;
-  if (ninputs == 0) return hipSuccess;
-  const uint32_t nl = (uint32_t)__builtin_popcount(limb_mask);
-  if (nl == 0 || limb_mask >> L || (dot.mask & ~limb_mask)) return hipErrorInvalidValue;
-  // the split kernels also serve limb subsets and D (k_encrypt_combine forms every limb of c0 and c1)
-  const bool split = use_split(logn, ninputs * 3 * nl) || ((nl != L || dot.mask) && encrypt_limbs_supported(logn));
-  if (split && a.jobs && a.load == NTT_LOAD_ENC && a.store == NTT_STORE_NONE) {
-    *combined = true;
-    return launch_encrypt_split(logn, a, ninputs, L, limb_mask, dot, pkp, cts, s);
-  }
-  if (nl != L || dot.mask) return hipErrorInvalidValue;  // k_encrypt_combine forms every limb, no D
-  return launch_ntt(logn, false, a, ninputs * 3 * L, s);
-}
-
-hipError_t launch_ntt(int logn, bool inverse, const NttArgs& a, uint32_t njobs, hipStream_t s) {
-  if (njobs == 0) return hipSuccess;
-  const bool segsum = a.jobs && a.store == NTT_STORE_SEGSUM;
-  if (segsum && (!inverse || whole_unavailable(logn, njobs) || logn > NTT_WHOLE_MAX_LOGN || a.cols < 1 ||
-                 a.cols > NTT_SEGSUM_FUSED_MAX_COLS))
-    return hipErrorInvalidValue;  // the segment-sum epilogue exists in the whole-polynomial inverse only
-  if (!segsum && use_split(logn, njobs)) return launch_ntt_split(logn, inverse, a, njobs, s);
+template <class BIG>
+hipError_t launch_ntt_whole(int logn, bool inverse, const NttArgs& a, uint32_t njobs, hipStream_t s) {
 #define TH_NTT_CASE(L) \
-  case L: return inverse ? launch_one<L, true>(a, njobs, s) : launch_one<L, false>(a, njobs, s);
+  case L: return inverse ? launch_one<BIG, L, true>(a, njobs, s) : launch_one<BIG, L, false>(a, njobs, s);
   switch (logn) {
     TH_NTT_CASE(10)
     TH_NTT_CASE(11)
@@ -514,5 +439,10 @@ hipError_t launch_ntt(int logn, bool inverse, const NttArgs& a, uint32_t njobs, 
   }
 #undef TH_NTT_CASE
 }
+
+// The launchers for this object's arithmetic (the Makefile compiles this file
+// once per TH_BIG).
+template hipError_t launch_ntt_whole<TH_BIG>(int, bool, const NttArgs&, uint32_t, hipStream_t);
+template hipError_t launch_rescale_decrypt_whole<TH_BIG>(int, const RescaleDecryptArgs&, uint32_t, hipStream_t);
 
 }  // namespace th

@@ -38,7 +38,9 @@
 // natural layout; they are given workgroup ids that the dispatcher sends to
 // the same XCD (ids are dealt round-robin over the 8 XCDs), so the second
 // half of each line is served by that XCD's L2.
+// The kernels are templates of the chain's arithmetic above 2^41 (BIG).
 #include "ntt_arith.h"
+#include "ntt_kernels.h"
 
 namespace th {
 
@@ -75,7 +77,9 @@ __device__ __forceinline__ uint32_t pad16(uint32_t e) { return e + (e >> 4); }
 // against 36.1 us).
 // The twiddles come from get(b, base, s): entry base | s of stage b's table
 // (s = the slot of the register pair among the stage's twiddles of the lane).
-template <int LOGN, int EB, int BHI, int BLO, class A, bool BATCH, class Get>
+// FRESH: the values are as loaded (below 4q), not a pass's output, so the
+// first stage folds nothing (PmArith).
+template <int LOGN, int EB, int BHI, int BLO, class A, bool BATCH, bool FRESH = false, class Get>
 __device__ __forceinline__ void fwd_stages_get(typename A::V (&x)[16], uint32_t f, const Get& get, const A& ar) {
 #pragma unroll
   for (int b = BHI; b >= BLO; --b) {
@@ -91,14 +95,14 @@ __device__ __forceinline__ void fwd_stages_get(typename A::V (&x)[16], uint32_t 
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (k & (1 << rb)) continue;
-        ar.fwd(x[k], x[k | (1 << rb)], t[k >> (rb + 1)]);
+        ar.fwd(x[k], x[k | (1 << rb)], t[k >> (rb + 1)], !FRESH && b == BHI);
       }
     } else {
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (k & (1 << rb)) continue;
         const typename A::Tw t = get(b, base, (uint32_t)(k >> (rb + 1)));
-        ar.fwd(x[k], x[k | (1 << rb)], t);
+        ar.fwd(x[k], x[k | (1 << rb)], t, !FRESH && b == BHI);
       }
     }
   }
@@ -117,6 +121,7 @@ __device__ __forceinline__ void fwd_stages(typename A::V (&x)[16], uint32_t f, G
 template <int LOGN, int EB, int BLO, int BHI, class A, bool BATCH, class Get>
 __device__ __forceinline__ void inv_stages_get(typename A::V (&x)[16], uint32_t f, const Get& get, const A& ar,
                                                const LimbConst& lc) {
+  constexpr InvPlan<BLO - EB, BHI - BLO + 1> plan;
 #pragma unroll
   for (int b = BLO; b <= BHI; ++b) {
     const int rb = b - EB;
@@ -134,13 +139,14 @@ __device__ __forceinline__ void inv_stages_get(typename A::V (&x)[16], uint32_t 
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int k = 0; k < 16; ++k)
-        if (!(k & (1 << rb))) ar.inv(x[k], x[k | (1 << rb)], t[k >> (rb + 1)]);
+        if (!(k & (1 << rb)))
+          ar.inv(x[k], x[k | (1 << rb)], t[k >> (rb + 1)], plan.small[b - BLO][k], plan.fold[b - BLO][k]);
     } else {
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (k & (1 << rb)) continue;
         const typename A::Tw t = get(b, base, (uint32_t)(k >> (rb + 1)));
-        ar.inv(x[k], x[k | (1 << rb)], t);
+        ar.inv(x[k], x[k | (1 << rb)], t, plan.small[b - BLO][k], plan.fold[b - BLO][k]);
       }
     }
   }
@@ -246,7 +252,7 @@ __device__ __forceinline__ void column_fwd_regs(typename A::V (&x)[16], uint64_t
   const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd));
   // stages on bits >= LOGN - 4 (the Q1 registers): every lane's element
   // bits above the stage are zero, so the twiddle index is uniform (f = 0)
-  fwd_stages_get<LOGN, LOGN - 4, LOGN - 1, LOGN - 4, A, BATCH>(
+  fwd_stages_get<LOGN, LOGN - 4, LOGN - 1, LOGN - 4, A, BATCH, true>(
       x, 0u, [&](int, uint32_t base, uint32_t s) { return ld16_uniform(tw, base | s); }, ar);
   exchange_in<HALF>(x, lds_raw, [&](uint32_t k) { return m.e1(k); }, [&](uint32_t k) { return m.e2(k); });
   fwd_stages<LOGN, CB, LOGN - 5, CB, A, BATCH>(x, m.j2(0), tw, ar);
@@ -287,10 +293,10 @@ __device__ __forceinline__ void column_pass(const uint64_t* __restrict__ src, ui
       op.fetch16(src, [&](int k) { return m.j1(k); }, r);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = ar.load(op.finish(r[k]));
+      for (int k = 0; k < 16; ++k) x[k] = ar.load(op.template finish<A>(r[k]));
     } else {
 #pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = ar.load(op(src, m.j1(k)));
+      for (int k = 0; k < 16; ++k) x[k] = ar.load(op.template at<A>(src, m.j1(k)));
     }
     column_fwd_regs<LOGN, A, false, true>(x, dst, lc, m, ar, lds_raw);
   } else {
@@ -462,7 +468,7 @@ __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint6
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = ar.load(op.finish(r[k]));
+      for (int k = 0; k < 16; ++k) x[k] = ar.load(op.template finish<A>(r[k]));
       // the second register pass's twiddles (stages 4 .. CB - 1) staged once
       // per wavefront in LDS; the exchanges' barriers order the staging
       const RowStage<LOGN, typename A::Tw> st(reinterpret_cast<typename A::Tw*>(lds_raw + S::LDS), jbase);
@@ -473,7 +479,7 @@ __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint6
       inv_stages_get<LOGN, CB - 4, 4, CB - 1, A, true>(x, jbase + p1(0), st, ar, lc);
     } else {
 #pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = ar.load(op(src, jbase + g(k)));
+      for (int k = 0; k < 16; ++k) x[k] = ar.load(op.template at<A>(src, jbase + g(k)));
       wave_exchange(x, lds, g, p2);
       inv_stages_get<LOGN, 0, 0, 3, A, true>(x, jbase + p2(0), row_get(lc.inv_row), ar, lc);
       wave_exchange(x, lds, p2, p1);
@@ -503,7 +509,7 @@ __device__ __forceinline__ uint32_t column_part(uint32_t p) {
 // the transform's input applies the fused load operation and the forward
 // row pass the fused store operation; otherwise passes read and write the
 // destination only.
-template <int LOGN, bool INV, bool COLUMN, uint32_t LD, uint32_t ST>
+template <class BIG, int LOGN, bool INV, bool COLUMN, uint32_t LD, uint32_t ST>
 __global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
   using S = Split<LOGN>;
   // the forward row pass with a fused rescale store, and the inverse row pass
@@ -535,17 +541,12 @@ __global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
     limb = a.limb_base + job % a.limb_mod;
   }
   const LimbConst& lc = a.lc[limb];
-  if constexpr (COLUMN) {
-    if (lc.fp64)
-      column_pass<LOGN, INV, Fp64Arith>(src, dst, lc, op, part, lds);
+  with_arith<BIG>(lc, [&]<class A>() {
+    if constexpr (COLUMN)
+      column_pass<LOGN, INV, A>(src, dst, lc, op, part, lds);
     else
-      column_pass<LOGN, INV, IntArith>(src, dst, lc, op, part, lds);
-  } else {
-    if (lc.fp64)
-      row_pass<LOGN, INV, Fp64Arith>(src, dst, lc, op, so, part, lds);
-    else
-      row_pass<LOGN, INV, IntArith>(src, dst, lc, op, so, part, lds);
-  }
+      row_pass<LOGN, INV, A>(src, dst, lc, op, so, part, lds);
+  });
 }
 
 // Rescale column kernel: the column pass that ends the inverse transform of a
@@ -561,7 +562,7 @@ __global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
 // forward passes (workgroup b: part b % PARTS of forward job b / PARTS), so
 // the launch takes one inverse and one forward pass instead of the inverse
 // and nf forward passes in turn.
-template <int LOGN>
+template <class BIG, int LOGN>
 __global__ __launch_bounds__(64) void rescale_column_kernel(NttArgs inv, NttArgs fwd, uint32_t nf, uint32_t fan) {
   using S = Split<LOGN>;
   __shared__ uint64_t lds[S::LDS];
@@ -572,20 +573,15 @@ __global__ __launch_bounds__(64) void rescale_column_kernel(NttArgs inv, NttArgs
   const NttJob ij = inv.jobs[job];
   const LimbConst& lci = inv.lc[ij.limb];
   uint64_t c[16];  // canonical last-limb coefficients of this wavefront's columns (Q1)
-  if (lci.fp64) {
-    const Fp64Arith ar(lci);
-    Fp64Arith::V x[16];
+  with_arith<BIG>(lci, [&]<class A>() {
+    const A ar(lci);
+    typename A::V x[16];
     column_inv_regs<LOGN>(x, ij.dst, lci, m, ar, lds);
 #pragma unroll
     for (int k = 0; k < 16; ++k) c[k] = ar.inv_store(x[k]);
-  } else {
-    const IntArith ar(lci);
-    IntArith::V x[16];
-    column_inv_regs<LOGN>(x, ij.dst, lci, m, ar, lds);
-#pragma unroll
-    for (int k = 0; k < 16; ++k) c[k] = ar.inv_store(x[k]);
-  }
-  // c mod q_l: FP64 on limbs below 2^41, else Barrett when c >= q_l
+  });
+  // c mod q_l: FP64 on limbs below 2^41, as it is on pm limbs (c < 2^61 < 3q),
+  // else Barrett when c >= q_l
   for (uint32_t f = f0; f < f1; ++f) {
     const NttJob fj = fwd.jobs[(uint64_t)job * nf + f];
     const LimbConst& lcf = fwd.lc[fj.limb];
@@ -594,19 +590,20 @@ __global__ __launch_bounds__(64) void rescale_column_kernel(NttArgs inv, NttArgs
     // hoisting per-coefficient terms out of the loop into extra registers
 #pragma unroll
     for (int k = 0; k < 16; ++k) c[k] = opaque_u64(c[k]);
-    if (lcf.fp64) {
-      const Fp64Arith ar(lcf);
-      Fp64Arith::V x[16];
+    with_arith<BIG>(lcf, [&]<class A>() {
+      const A ar(lcf);
+      typename A::V x[16];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = reduce_u64_f64(c[k], rc);
-      column_fwd_regs<LOGN, Fp64Arith, true>(x, fj.dst, lcf, m, ar, lds);
-    } else {
-      const IntArith ar(lcf);
-      IntArith::V x[16];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = c[k] < rc.q ? c[k] : mulmod_barrett(c[k], 1, rc.b);
-      column_fwd_regs<LOGN, IntArith, true>(x, fj.dst, lcf, m, ar, lds);
-    }
+      for (int k = 0; k < 16; ++k) {
+        if constexpr (std::is_same_v<A, Fp64Arith>)
+          x[k] = reduce_u64_f64(c[k], rc);
+        else if constexpr (std::is_same_v<A, PmArith>)
+          x[k] = c[k];
+        else
+          x[k] = c[k] < rc.q ? c[k] : mulmod_barrett(c[k], 1, rc.b);
+      }
+      column_fwd_regs<LOGN, A, true>(x, fj.dst, lcf, m, ar, lds);
+    });
   }
 }
 
@@ -614,13 +611,13 @@ __global__ __launch_bounds__(64) void rescale_column_kernel(NttArgs inv, NttArgs
 // wavefronts (3 per SIMD at its registers, 1024 SIMDs).
 constexpr uint32_t RESCALE_FAN_MAX_WAVES = 3072;
 
-template <int LOGN>
+template <class BIG, int LOGN>
 static hipError_t launch_rescale_t(const NttArgs& inv, uint32_t ninv, const NttArgs& fwd, uint32_t nf, hipStream_t s) {
   using S = Split<LOGN>;
   const dim3 block(64);
   const hipError_t e = with_ops<true>(inv.load, inv.store, [&]<uint32_t LD, uint32_t ST>() -> hipError_t {
     if constexpr (ST != NTT_STORE_NONE) return hipErrorInvalidValue;  // segment sums: whole kernel only
-    hipLaunchKernelGGL((ntt_split_kernel<LOGN, true, false, LD, NTT_STORE_NONE>), dim3(ninv * S::PARTS), block, 0, s,
+    hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, false, LD, NTT_STORE_NONE>), dim3(ninv * S::PARTS), block, 0, s,
                        inv);
     return hipGetLastError();
   });
@@ -628,23 +625,24 @@ static hipError_t launch_rescale_t(const NttArgs& inv, uint32_t ninv, const NttA
   // a batch whose nf passes per inverse job would leave most SIMDs idle
   // fans them out (RESCALE_FAN_MAX_WAVES)
   const uint32_t fan = ninv * nf * S::PARTS <= RESCALE_FAN_MAX_WAVES ? 1u : 0u;
-  hipLaunchKernelGGL((rescale_column_kernel<LOGN>), dim3(ninv * S::PARTS * (fan ? nf : 1)), block, 0, s, inv, fwd, nf,
+  hipLaunchKernelGGL((rescale_column_kernel<BIG, LOGN>), dim3(ninv * S::PARTS * (fan ? nf : 1)), block, 0, s, inv, fwd, nf,
                      fan);
   const hipError_t e2 = hipGetLastError();
   if (e2 != hipSuccess) return e2;
   return with_ops<false>(fwd.load, fwd.store, [&]<uint32_t LD, uint32_t ST>() -> hipError_t {
-    hipLaunchKernelGGL((ntt_split_kernel<LOGN, false, false, NTT_LOAD_NONE, ST>), dim3(ninv * nf * S::PARTS), block, 0,
+    hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, false, NTT_LOAD_NONE, ST>), dim3(ninv * nf * S::PARTS), block, 0,
                        s, fwd);
     return hipGetLastError();
   });
 }
 
+template <class BIG>
 hipError_t launch_rescale_split(int logn, const NttArgs& inv, uint32_t ninv, const NttArgs& fwd, uint32_t nf,
                                 hipStream_t s) {
   switch (logn) {
-    case 13: return launch_rescale_t<13>(inv, ninv, fwd, nf, s);
-    case 14: return launch_rescale_t<14>(inv, ninv, fwd, nf, s);
-    case 15: return launch_rescale_t<15>(inv, ninv, fwd, nf, s);
+    case 13: return launch_rescale_t<BIG, 13>(inv, ninv, fwd, nf, s);
+    case 14: return launch_rescale_t<BIG, 14>(inv, ninv, fwd, nf, s);
+    case 15: return launch_rescale_t<BIG, 15>(inv, ninv, fwd, nf, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -656,7 +654,8 @@ hipError_t launch_rescale_split(int logn, const NttArgs& inv, uint32_t ninv, con
 // so the three transforms are never written out. Workgroup w works on part
 // w % PARTS of input / limb w / PARTS with three wavefronts, one per
 // transform (0: M, 1: U, 2: E1), each with its own LDS slice; U's wavefront
-// hands its canonical outputs to the other two through LDS, which form and
+// hands its outputs to the other two through LDS (canonical, except on pm
+// limbs, whose products take any 64-bit value), which form and
 // store c0 and c1. The limbs are those in mask (n of them); jobs: 3n per
 // input (M, E1 and U of each of those limbs in increasing order);
 // pkp = [b (L) | a (L)] as prepared pairs (w, companion), so each product is
@@ -664,7 +663,7 @@ hipError_t launch_rescale_split(int logn, const NttArgs& inv, uint32_t ninv, con
 // in dot.mask the kernel stores D = c0 + c1 s instead (EncDot): M's and E1's
 // wavefronts each hand the other half of their outputs over through LDS and
 // form D on their own half.
-template <int LOGN>
+template <class BIG, int LOGN>
 __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint64_t* pkp, uint64_t* cts, uint32_t L,
                                                           uint32_t mask, EncDot dot) {
   using S = Split<LOGN>;
@@ -697,7 +696,7 @@ __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint6
     }
     if (wv == 1) {
 #pragma unroll
-      for (int k = 0; k < 16; ++k) shared_u[lane + 64 * k] = ar.fwd_store(x[k]);
+      for (int k = 0; k < 16; ++k) shared_u[lane + 64 * k] = std::is_same_v<A, PmArith> ? ar.raw(x[k]) : ar.fwd_store(x[k]);
     }
     __syncthreads();
     uint64_t c[16];  // M's and E1's wavefronts keep c0, c1 where D is formed
@@ -705,17 +704,19 @@ __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint6
       const GMut<uint64_t> out = gst(cts + (size_t)i * 2 * L * S::N + (wv == 0 ? 0 : (size_t)L * S::N)) + off;
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
-        const uint64_t u = shared_u[lane + 64 * k], m = ar.fwd_store(x[k]);
+        const uint64_t u = shared_u[lane + 64 * k];
         const ShoupTw p = kp[k];
         uint64_t r;
         if constexpr (std::is_same_v<A, Fp64Arith>) {
           // (-q/2, q/2) + [0, q)
           double t = mulmod_f64(u64_to_f64(u), u64_to_f64(p.w), __builtin_bit_cast(double, p.ws), lc.qd) +
-                     u64_to_f64(m);
+                     u64_to_f64(ar.fwd_store(x[k]));
           t = t < 0.0 ? t + lc.qd : t;
           r = f64_to_u64(t >= lc.qd ? t - lc.qd : t);
+        } else if constexpr (std::is_same_v<A, PmArith>) {
+          r = pm_canon(pm_mul_fixed(u, __builtin_bit_cast(PmTw, p), ar.c2) + pm_fold(x[k], ar.c), bc.q, ar.c);
         } else {
-          r = shoup_approx(u, p.w, p.ws, bc.q) + m;  // [0, 5q)
+          r = shoup_approx(u, p.w, p.ws, bc.q) + ar.fwd_store(x[k]);  // [0, 5q)
           r = csub(csub(csub(r, 4 * bc.q), 2 * bc.q), bc.q);
         }
         if (!form_d) {
@@ -730,7 +731,7 @@ __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint6
       }
     }
     if (form_d) {
-      // D = c0 + c1 s in [0, 3q) (the key in Montgomery form), at input i's
+      // D = c0 + c1 s in [0, 3q) (the key prepared for fixed_mul), at input i's
       // slot for this limb: the position of l among dot.mask's limbs
       const uint32_t kd = (uint32_t)__builtin_popcount(dot.mask & ((1u << l) - 1));
       const uint32_t nd = (uint32_t)__builtin_popcount(dot.mask);
@@ -745,37 +746,35 @@ __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint6
       __syncthreads();
       if (wv == 0) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) dst[64 * k] = c[k] + mont_mul(lds[2][lane + 64 * k], sv[k], bc);
+        for (int k = 0; k < 8; ++k) dst[64 * k] = key_dot<A>(c[k], lds[2][lane + 64 * k], sv[k], bc);
       } else if (wv == 2) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) dst[64 * (8 + k)] = lds[2][lane + 64 * (8 + k)] + mont_mul(c[8 + k], sv[k], bc);
+        for (int k = 0; k < 8; ++k) dst[64 * (8 + k)] = key_dot<A>(lds[2][lane + 64 * (8 + k)], c[8 + k], sv[k], bc);
       }
     }
   };
-  if (lc.fp64)
-    run.template operator()<Fp64Arith>();
-  else
-    run.template operator()<IntArith>();
+  with_arith<BIG>(lc, run);
 }
 
-template <int LOGN>
+template <class BIG, int LOGN>
 static hipError_t launch_encrypt_t(const NttArgs& a, uint32_t ninputs, uint32_t L, uint32_t mask, const EncDot& dot,
                                    const uint64_t* pkp, uint64_t* cts, hipStream_t s) {
   using S = Split<LOGN>;
   const uint32_t nl = (uint32_t)__builtin_popcount(mask);
-  hipLaunchKernelGGL((ntt_split_kernel<LOGN, false, true, NTT_LOAD_ENC, NTT_STORE_NONE>),
+  hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, true, NTT_LOAD_ENC, NTT_STORE_NONE>),
                      dim3(ninputs * 3 * nl * S::PARTS), dim3(64), 0, s, a);
-  hipLaunchKernelGGL((encrypt_row_kernel<LOGN>), dim3(ninputs * nl * S::PARTS), dim3(192), 0, s, a, pkp, cts, L,
+  hipLaunchKernelGGL((encrypt_row_kernel<BIG, LOGN>), dim3(ninputs * nl * S::PARTS), dim3(192), 0, s, a, pkp, cts, L,
                      mask, dot);
   return hipGetLastError();
 }
 
+template <class BIG>
 hipError_t launch_encrypt_split(int logn, const NttArgs& a, uint32_t ninputs, uint32_t L, uint32_t limb_mask,
                                 const EncDot& dot, const uint64_t* pkp, uint64_t* cts, hipStream_t s) {
   switch (logn) {
-    case 13: return launch_encrypt_t<13>(a, ninputs, L, limb_mask, dot, pkp, cts, s);
-    case 14: return launch_encrypt_t<14>(a, ninputs, L, limb_mask, dot, pkp, cts, s);
-    case 15: return launch_encrypt_t<15>(a, ninputs, L, limb_mask, dot, pkp, cts, s);
+    case 13: return launch_encrypt_t<BIG, 13>(a, ninputs, L, limb_mask, dot, pkp, cts, s);
+    case 14: return launch_encrypt_t<BIG, 14>(a, ninputs, L, limb_mask, dot, pkp, cts, s);
+    case 15: return launch_encrypt_t<BIG, 15>(a, ninputs, L, limb_mask, dot, pkp, cts, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -783,7 +782,7 @@ hipError_t launch_encrypt_split(int logn, const NttArgs& a, uint32_t ninputs, ui
 // The pass that reads the transform's input (column pass forward, row pass
 // inverse) carries the load operation, the forward row pass the store
 // operation; the other pass is instantiated with none.
-template <int LOGN, bool INV>
+template <class BIG, int LOGN, bool INV>
 static hipError_t launch_split_t(const NttArgs& a, uint32_t njobs, hipStream_t s) {
   using S = Split<LOGN>;
   const dim3 grid(njobs * S::PARTS), block(64);
@@ -791,25 +790,26 @@ static hipError_t launch_split_t(const NttArgs& a, uint32_t njobs, hipStream_t s
                        [&]<uint32_t LD, uint32_t ST>() -> hipError_t {
                          if constexpr (ST == NTT_STORE_SEGSUM) return hipErrorInvalidValue;  // whole kernel only
                          if constexpr (!INV) {
-                           hipLaunchKernelGGL((ntt_split_kernel<LOGN, false, true, LD, NTT_STORE_NONE>), grid, block,
+                           hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, true, LD, NTT_STORE_NONE>), grid, block,
                                               0, s, a);
-                           hipLaunchKernelGGL((ntt_split_kernel<LOGN, false, false, NTT_LOAD_NONE, ST>), grid, block,
+                           hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, false, NTT_LOAD_NONE, ST>), grid, block,
                                               0, s, a);
                          } else {
-                           hipLaunchKernelGGL((ntt_split_kernel<LOGN, true, false, LD, NTT_STORE_NONE>), grid, block,
+                           hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, false, LD, NTT_STORE_NONE>), grid, block,
                                               0, s, a);
-                           hipLaunchKernelGGL((ntt_split_kernel<LOGN, true, true, NTT_LOAD_NONE, NTT_STORE_NONE>), grid,
+                           hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, true, NTT_LOAD_NONE, NTT_STORE_NONE>), grid,
                                               block, 0, s, a);
                          }
                          return hipGetLastError();
                        });
 }
 
+template <class BIG>
 hipError_t launch_ntt_split(int logn, bool inverse, const NttArgs& a, uint32_t njobs, hipStream_t s) {
   switch (logn) {
-    case 13: return inverse ? launch_split_t<13, true>(a, njobs, s) : launch_split_t<13, false>(a, njobs, s);
-    case 14: return inverse ? launch_split_t<14, true>(a, njobs, s) : launch_split_t<14, false>(a, njobs, s);
-    case 15: return inverse ? launch_split_t<15, true>(a, njobs, s) : launch_split_t<15, false>(a, njobs, s);
+    case 13: return inverse ? launch_split_t<BIG, 13, true>(a, njobs, s) : launch_split_t<BIG, 13, false>(a, njobs, s);
+    case 14: return inverse ? launch_split_t<BIG, 14, true>(a, njobs, s) : launch_split_t<BIG, 14, false>(a, njobs, s);
+    case 15: return inverse ? launch_split_t<BIG, 15, true>(a, njobs, s) : launch_split_t<BIG, 15, false>(a, njobs, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -839,9 +839,8 @@ hipError_t launch_ntt_split(int logn, bool inverse, const NttArgs& a, uint32_t n
 
 // Step 2. Workgroup w: part w % PARTS of inverse job w / PARTS (jobs 2b, 2b+1
 // = X, Y of batch b; their dst holds step 1's intermediate).
-template <int LOGN>
-__global__ __launch_bounds__(64) void rd_column_kernel(NttArgs inv, const RescaleConst* __restrict__ rc0,
-                                                       const LimbConst* __restrict__ lc0p) {
+template <class BIG, int LOGN>
+__global__ __launch_bounds__(64) void rd_column_kernel(NttArgs inv, const RescaleConst* __restrict__ rc0) {
   using S = Split<LOGN>;
   __shared__ uint64_t lds[S::LDS];
   const uint32_t job = blockIdx.x / S::PARTS;
@@ -850,47 +849,38 @@ __global__ __launch_bounds__(64) void rd_column_kernel(NttArgs inv, const Rescal
   const LimbConst& lci = inv.lc[ij.limb];
   const RescaleConst rc = *rc0;
   uint64_t c[16];  // the last limb's canonical coefficients, then reduced mod q0
-  if (lci.fp64) {
-    const Fp64Arith ar(lci);
-    Fp64Arith::V x[16];
+  with_arith<BIG>(lci, [&]<class A>() {
+    const A ar(lci);
+    typename A::V x[16];
     column_inv_regs<LOGN>(x, ij.dst, lci, m, ar, lds);
 #pragma unroll
     for (int k = 0; k < 16; ++k) c[k] = ar.inv_store(x[k]);
-  } else {
-    const IntArith ar(lci);
-    IntArith::V x[16];
-    column_inv_regs<LOGN>(x, ij.dst, lci, m, ar, lds);
+  });
+  // pm limbs take it as it is (below 2^61 < 3q)
+  const LimbConst& lc0 = inv.lc[0];
+  if (lc0.kind == LIMB_FP64 || std::is_same_v<BIG, IntArith>) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) c[k] = ar.inv_store(x[k]);
+    for (int k = 0; k < 16; ++k) c[k] = c[k] < rc.q ? c[k] : mulmod_barrett(c[k], 1, rc.b);
   }
-#pragma unroll
-  for (int k = 0; k < 16; ++k) c[k] = c[k] < rc.q ? c[k] : mulmod_barrett(c[k], 1, rc.b);
   if ((job & 1) == 0) {
     const GMut<uint64_t> out = gst(ij.dst);
 #pragma unroll
     for (int k = 0; k < 16; ++k) out[m.j1(k)] = c[k];  // r0, natural order
     return;
   }
-  const LimbConst& lc0 = *lc0p;
-  if (lc0.fp64) {
-    const Fp64Arith ar(lc0);
-    Fp64Arith::V x[16];
+  with_arith<BIG>(lc0, [&]<class A>() {
+    const A ar(lc0);
+    typename A::V x[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.load(c[k]);
-    column_fwd_regs<LOGN, Fp64Arith, true>(x, ij.dst, lc0, m, ar, lds);
-  } else {
-    const IntArith ar(lc0);
-    IntArith::V x[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = ar.load(c[k]);
-    column_fwd_regs<LOGN, IntArith, true>(x, ij.dst, lc0, m, ar, lds);
-  }
+    column_fwd_regs<LOGN, A, true>(x, ij.dst, lc0, m, ar, lds);
+  });
 }
 
 // Step 3. Workgroup w: part w % PARTS of batch w / PARTS (RescaleDecryptJob:
 // y holds step 2's forward column intermediate; rewritten in place with the
 // inverse row pass's intermediate of D pt - NTT(r1) s).
-template <int LOGN>
+template <class BIG, int LOGN>
 __global__ __launch_bounds__(64) void rd_row_kernel(RescaleDecryptArgs a) {
   using S = Split<LOGN>;
   constexpr int CB = S::CB, M = (1 << (CB - 4)) - 1;
@@ -911,19 +901,12 @@ __global__ __launch_bounds__(64) void rd_row_kernel(RescaleDecryptArgs a) {
     typename A::V* lds = reinterpret_cast<typename A::V*>(lds_raw);
     row_fwd_regs<LOGN>(x, jb.y, lc, ar, part, lds_raw);
     {
-      // D pt - NTT(r1) s at positions jbase + g(k): Montgomery products, each
-      // in [0, 2q), so the difference plus 2q is in (0, 4q), the integer
-      // inverse's input range; the FP64 inverse gets it canonical
+      // D pt - NTT(r1) s at positions jbase + g(k)
       const GPtr<uint64_t> d = gld(jb.d), p = gld(jb.ptm), sk = gld(a.skm);
-      const uint64_t q = lc.q, two_q = 2 * lc.q;
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         const uint32_t i = jbase + g(k);
-        const uint64_t u = mont_mul(d[i], p[i], bc);
-        const uint64_t t = mont_mul(ar.fwd_store(x[k]), sk[i], bc);
-        uint64_t e = u + two_q - t;
-        if constexpr (std::is_same_v<A, Fp64Arith>) e = csub(csub(e, two_q), q);
-        x[k] = ar.load(e);
+        x[k] = ar.load(prepared_difference(ar, d[i], p[i], x[k], sk[i], bc));
       }
     }
     const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.inv));
@@ -938,17 +921,14 @@ __global__ __launch_bounds__(64) void rd_row_kernel(RescaleDecryptArgs a) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) out[jbase + p1(k)] = ar.raw(x[k]);
   };
-  if (lc.fp64)
-    run.template operator()<Fp64Arith>();
-  else
-    run.template operator()<IntArith>();
+  with_arith<BIG>(lc, run);
 }
 
 // Step 4. Workgroup w: column part w % PARTS of batch w / PARTS; writes
 // lane t's sums for segments c < cols at partials + (b cols + c) T + t,
 // T = 2^(LOGN-4). Without RESCALED (a plain decryption, launch_decrypt_sums_split)
 // the decrypted coefficient is the transform's output itself.
-template <int LOGN, bool RESCALED = true>
+template <class BIG, int LOGN, bool RESCALED = true>
 __global__ __launch_bounds__(64) void rd_column_sums_kernel(RescaleDecryptArgs a, double* __restrict__ partials) {
   using S = Split<LOGN>;
   constexpr int MAXC = NTT_SEGSUM_FUSED_MAX_COLS;
@@ -960,30 +940,27 @@ __global__ __launch_bounds__(64) void rd_column_sums_kernel(RescaleDecryptArgs a
   const LimbConst& lc = a.lc[0];
   const RescaleConst rc = RESCALED ? *a.rc : RescaleConst{};
   const uint64_t q = lc.q, half = q >> 1;
+  const GPtr<uint64_t> r0 = gld(RESCALED ? jb.x : jb.y);
   uint64_t mv[16];
-  if (lc.fp64) {
-    const Fp64Arith ar(lc);
-    Fp64Arith::V x[16];
+  with_arith<BIG>(lc, [&]<class A>() {
+    const A ar(lc);
+    typename A::V x[16];
     column_inv_regs<LOGN>(x, jb.y, lc, m, ar, lds);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) mv[k] = ar.inv_store(x[k]);
-  } else {
-    const IntArith ar(lc);
-    IntArith::V x[16];
-    column_inv_regs<LOGN>(x, jb.y, lc, m, ar, lds);
-#pragma unroll
-    for (int k = 0; k < 16; ++k) mv[k] = ar.inv_store(x[k]);
-  }
+    for (int k = 0; k < 16; ++k) {
+      mv[k] = ar.inv_store(x[k]);
+      if constexpr (RESCALED) mv[k] = rescaled_coefficient<A>(mv[k], r0[m.j1(k)], rc, lc);
+    }
+  });
   using D2 = double __attribute__((ext_vector_type(2)));
   const GPtr<D2> W = gld(reinterpret_cast<const D2*>(a.segw));
-  const GPtr<uint64_t> r0 = gld(RESCALED ? jb.x : jb.y);
   double acc[MAXC];
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) acc[c] = 0.0;
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
     const uint32_t j = m.j1(k);
-    const uint64_t v0 = RESCALED ? csub(shoup_lazy(submod(mv[k], r0[j], q), rc.inv, rc.inv_s, q), q) : mv[k];
+    const uint64_t v0 = mv[k];
     const double v = v0 > half ? -(double)(q - v0) : (double)v0;
     const D2 p = W[j];  // W_0[j], 2 cos(2 phi_j)
     double wp = p.x, wc = p.x;
@@ -1008,7 +985,7 @@ __global__ __launch_bounds__(64) void rd_column_sums_kernel(RescaleDecryptArgs a
 // Step 5. One wavefront per batch and segment: the sum over groups of 64
 // consecutive lanes t by a butterfly tree, the groups added in order (every
 // group's values requested first, the trees independent of one another).
-template <int LOGN>
+template <class BIG, int LOGN>
 __global__ __launch_bounds__(64) void rd_sums_final_kernel(RescaleDecryptArgs a, const double* __restrict__ partials) {
   constexpr uint32_t T = 1u << (LOGN - 4), G = T / 64;
   const uint32_t b = blockIdx.x / a.cols, c = blockIdx.x % a.cols, lane = threadIdx.x;
@@ -1027,59 +1004,72 @@ __global__ __launch_bounds__(64) void rd_sums_final_kernel(RescaleDecryptArgs a,
   if (lane == 0) gst(jb.seg)[c] = t / jb.scale;
 }
 
-template <int LOGN>
+template <class BIG, int LOGN>
 static hipError_t launch_rd_split_t(const NttArgs& inv, const RescaleDecryptArgs& a, uint32_t nb, double* partials,
                                     hipStream_t s) {
   using S = Split<LOGN>;
   const dim3 block(64);
-  hipLaunchKernelGGL((ntt_split_kernel<LOGN, true, false, NTT_LOAD_MULM, NTT_STORE_NONE>), dim3(2 * nb * S::PARTS),
+  hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, false, NTT_LOAD_MULM, NTT_STORE_NONE>), dim3(2 * nb * S::PARTS),
                      block, 0, s, inv);
-  hipLaunchKernelGGL((rd_column_kernel<LOGN>), dim3(2 * nb * S::PARTS), block, 0, s, inv, a.rc, a.lc);
-  hipLaunchKernelGGL((rd_row_kernel<LOGN>), dim3(nb * S::PARTS), block, 0, s, a);
-  hipLaunchKernelGGL((rd_column_sums_kernel<LOGN>), dim3(nb * S::PARTS), block, 0, s, a, partials);
-  hipLaunchKernelGGL((rd_sums_final_kernel<LOGN>), dim3(nb * a.cols), block, 0, s, a, (const double*)partials);
+  hipLaunchKernelGGL((rd_column_kernel<BIG, LOGN>), dim3(2 * nb * S::PARTS), block, 0, s, inv, a.rc);
+  hipLaunchKernelGGL((rd_row_kernel<BIG, LOGN>), dim3(nb * S::PARTS), block, 0, s, a);
+  hipLaunchKernelGGL((rd_column_sums_kernel<BIG, LOGN>), dim3(nb * S::PARTS), block, 0, s, a, partials);
+  hipLaunchKernelGGL((rd_sums_final_kernel<BIG, LOGN>), dim3(nb * a.cols), block, 0, s, a, (const double*)partials);
   return hipGetLastError();
 }
 
 // A plain batched decryption with segment sums on the split kernels: the
 // inverse row pass of c0 + c1 s (row: NTT_LOAD_DOTM jobs on limb 0, one per
 // batch, dst = the batch's y), then steps 4 and 5 without the rescale.
-template <int LOGN>
+template <class BIG, int LOGN>
 static hipError_t launch_dec_split_t(const NttArgs& row, const RescaleDecryptArgs& a, uint32_t nb, double* partials,
                                      hipStream_t s) {
   using S = Split<LOGN>;
   const dim3 block(64);
-  hipLaunchKernelGGL((ntt_split_kernel<LOGN, true, false, NTT_LOAD_DOTM, NTT_STORE_NONE>), dim3(nb * S::PARTS), block,
+  hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, false, NTT_LOAD_DOTM, NTT_STORE_NONE>), dim3(nb * S::PARTS), block,
                      0, s, row);
-  hipLaunchKernelGGL((rd_column_sums_kernel<LOGN, false>), dim3(nb * S::PARTS), block, 0, s, a, partials);
-  hipLaunchKernelGGL((rd_sums_final_kernel<LOGN>), dim3(nb * a.cols), block, 0, s, a, (const double*)partials);
+  hipLaunchKernelGGL((rd_column_sums_kernel<BIG, LOGN, false>), dim3(nb * S::PARTS), block, 0, s, a, partials);
+  hipLaunchKernelGGL((rd_sums_final_kernel<BIG, LOGN>), dim3(nb * a.cols), block, 0, s, a, (const double*)partials);
   return hipGetLastError();
 }
 
-hipError_t launch_decrypt_sums_split(int logn, const NttArgs& row, const RescaleDecryptArgs& a, uint32_t nb,
+template <class BIG>
+hipError_t launch_dec_split(int logn, const NttArgs& row, const RescaleDecryptArgs& a, uint32_t nb,
                                      double* partials, hipStream_t s) {
   if (nb == 0) return hipSuccess;
   if (!row.jobs || row.load != NTT_LOAD_DOTM || a.cols < 1 || a.cols > NTT_SEGSUM_FUSED_MAX_COLS)
     return hipErrorInvalidValue;
   switch (logn) {
-    case 13: return launch_dec_split_t<13>(row, a, nb, partials, s);
-    case 14: return launch_dec_split_t<14>(row, a, nb, partials, s);
-    case 15: return launch_dec_split_t<15>(row, a, nb, partials, s);
+    case 13: return launch_dec_split_t<BIG, 13>(row, a, nb, partials, s);
+    case 14: return launch_dec_split_t<BIG, 14>(row, a, nb, partials, s);
+    case 15: return launch_dec_split_t<BIG, 15>(row, a, nb, partials, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-hipError_t launch_rescale_decrypt_split(int logn, const NttArgs& inv, const RescaleDecryptArgs& a, uint32_t nb,
+template <class BIG>
+hipError_t launch_rd_split(int logn, const NttArgs& inv, const RescaleDecryptArgs& a, uint32_t nb,
                                         double* partials, hipStream_t s) {
   if (nb == 0) return hipSuccess;
   if (!inv.jobs || inv.load != NTT_LOAD_MULM || a.cols < 1 || a.cols > NTT_SEGSUM_FUSED_MAX_COLS)
     return hipErrorInvalidValue;
   switch (logn) {
-    case 13: return launch_rd_split_t<13>(inv, a, nb, partials, s);
-    case 14: return launch_rd_split_t<14>(inv, a, nb, partials, s);
-    case 15: return launch_rd_split_t<15>(inv, a, nb, partials, s);
+    case 13: return launch_rd_split_t<BIG, 13>(inv, a, nb, partials, s);
+    case 14: return launch_rd_split_t<BIG, 14>(inv, a, nb, partials, s);
+    case 15: return launch_rd_split_t<BIG, 15>(inv, a, nb, partials, s);
     default: return hipErrorInvalidValue;
   }
 }
+
+// The launchers for this object's arithmetic (the Makefile compiles this file
+// once per TH_BIG).
+template hipError_t launch_ntt_split<TH_BIG>(int, bool, const NttArgs&, uint32_t, hipStream_t);
+template hipError_t launch_rescale_split<TH_BIG>(int, const NttArgs&, uint32_t, const NttArgs&, uint32_t, hipStream_t);
+template hipError_t launch_encrypt_split<TH_BIG>(int, const NttArgs&, uint32_t, uint32_t, uint32_t, const EncDot&,
+                                                 const uint64_t*, uint64_t*, hipStream_t);
+template hipError_t launch_dec_split<TH_BIG>(int, const NttArgs&, const RescaleDecryptArgs&, uint32_t, double*,
+                                                      hipStream_t);
+template hipError_t launch_rd_split<TH_BIG>(int, const NttArgs&, const RescaleDecryptArgs&, uint32_t,
+                                                         double*, hipStream_t);
 
 }  // namespace th

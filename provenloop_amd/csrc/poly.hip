@@ -26,7 +26,7 @@ __global__ void k_ct_pt_mul(const CtPtJob* __restrict__ jobs, const BarrettConst
     const uint32_t w = e < per_comp ? e : e - per_comp;
     const uint32_t l = w / n;
     const uint64_t c = gld(e < per_comp ? jb.ct0 : jb.ct1)[w];
-    gst(jb.out)[e] = mulmod_barrett(c, gld(jb.pt)[w], bc[l]);
+    gst(jb.out)[e] = mulmod(c, gld(jb.pt)[w], bc[l]);
   }
 }
 
@@ -45,8 +45,8 @@ __global__ void k_ct_addsub(const AddJob* __restrict__ jobs, const uint64_t* __r
 
 // Operands fixed for many products (keys) prepared as pairs in the twiddle
 // tables' formats: (w, floor(w 2^64 / q)) on the integer limbs, (w, w / q as
-// a double) on limbs below 2^41, so a product by w is one Shoup or one FP64
-// step instead of a 64-bit Barrett reduction. src: count x L x n residues;
+// a double) on limbs below 2^41, PmTw on pm limbs, so a product by w is one
+// step of the transforms' kind instead of a 64-bit Barrett reduction. src: count x L x n residues;
 // dst: the same as 16-byte pairs.
 __device__ __forceinline__ uint64_t shoup_companion(uint64_t w, const BarrettConst& b) {
   // w 2^64 r / 2^128 with r = floor((2^128 - 1) / q) is at most 1 short of
@@ -66,8 +66,15 @@ __global__ void k_prepare_pairs(const uint64_t* __restrict__ src, uint64_t* __re
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t l = (uint32_t)((e / n) % L);
     const uint64_t w = src[e];
+    if (lc[l].kind == LIMB_PM) {
+      const uint64_t v = mulmod(w, 1ULL << 32, bc[l]);
+      constexpr uint32_t M30 = (1u << 30) - 1;
+      dst[2 * e] = (w & M30) | (w >> 30 << 32);
+      dst[2 * e + 1] = (v & M30) | (v >> 30 << 32);
+      continue;
+    }
     uint64_t c;
-    if (lc[l].fp64)
+    if (lc[l].kind == LIMB_FP64)
       c = __builtin_bit_cast(uint64_t, (double)w / lc[l].qd);  // correctly rounded: both exact below 2^53
     else
       c = shoup_companion(w, bc[l]);
@@ -76,12 +83,13 @@ __global__ void k_prepare_pairs(const uint64_t* __restrict__ src, uint64_t* __re
   }
 }
 
-// count x L x n residues into Montgomery form, w 2^64 mod q (mont_mul).
+// count x L x n residues prepared for prepared_mul and fixed_mul: into
+// Montgomery form, w 2^64 mod q (mont_mul); unchanged on pm limbs.
 __global__ void k_to_montgomery(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst,
                                 const BarrettConst* __restrict__ bc, uint32_t n, uint32_t L, uint64_t total) {
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (uint64_t)gridDim.x * blockDim.x) {
     const BarrettConst& m = bc[(e / n) % L];
-    dst[e] = csub(shoup_lazy(src[e], m.r64, m.r64_s, m.q), m.q);
+    dst[e] = m.pm_c ? src[e] : csub(shoup_lazy(src[e], m.r64, m.r64_s, m.q), m.q);
   }
 }
 
@@ -102,12 +110,12 @@ __global__ void k_sub_product(const uint64_t* __restrict__ x, const uint64_t* __
   const uint32_t total = L * n;
   for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
     const BarrettConst m = bc[e / n];
-    out[e] = submod(x[e], mulmod_barrett(a[e], s[e], m), m.q);
+    out[e] = submod(x[e], mulmod(a[e], s[e], m), m.q);
   }
 }
 
 // D = c0 + c1 s on limbs 0..nl-1 of count ciphertexts at cts + i ct_stride
-// ([c0 | c1], L limbs each), with the secret key in Montgomery form: the
+// ([c0 | c1], L limbs each), with the secret key prepared (k_to_montgomery): the
 // decryption's c0 + c1 s (ciphertext.rs:332-341), lazily in [0, 3q). For a
 // product ciphertext (c0 pt, c1 pt) the decryption is pt (c0 + c1 s), so one
 // D per input serves every plaintext it is multiplied by.
@@ -119,7 +127,9 @@ __global__ void k_key_dot(const uint64_t* __restrict__ cts, uint64_t ct_stride, 
     const uint64_t i = e / per, r = e - i * per;
     const uint32_t l = (uint32_t)(r / n);
     const uint64_t* c = cts + i * ct_stride;
-    out[e] = c[r] + mont_mul(c[(uint64_t)L * n + r], skm[r], bc[l]);
+    const BarrettConst m = bc[l];
+    const uint64_t d = c[r] + prepared_mul(c[(uint64_t)L * n + r], skm[r], m);
+    out[e] = m.pm_c ? pm_fold(d, (uint32_t)m.pm_c) : d;
   }
 }
 
@@ -137,8 +147,8 @@ __global__ void k_encrypt_combine(const EncCombineJob* __restrict__ jobs, const 
     const BarrettConst m = bc[l];
     const GPtr<uint64_t> prep = gld(jb.prep);
     const uint64_t U = prep[2 * total + e];
-    const uint64_t bu = mulmod_barrett(gld(jb.pk_b)[e], U, m);
-    const uint64_t au = mulmod_barrett(gld(jb.pk_a)[e], U, m);
+    const uint64_t bu = mulmod(gld(jb.pk_b)[e], U, m);
+    const uint64_t au = mulmod(gld(jb.pk_a)[e], U, m);
     gst(jb.out)[e] = addmod(bu, prep[e], m.q);
     gst(jb.out)[total + e] = addmod(au, prep[total + e], m.q);
   }

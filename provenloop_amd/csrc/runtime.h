@@ -205,7 +205,7 @@ struct th_ctx {
   uint32_t N = 0, logn = 0, L = 0;
   std::vector<uint64_t> q;
   std::vector<LimbConst> h_lc;
-  LimbConst* d_lc = nullptr;
+  LimbTable d_lc;
   BarrettConst* d_bc = nullptr;
   uint64_t* d_q = nullptr;
   RescaleConst* d_rc = nullptr;  // [level][l], level = input limb count (2..L), row stride L

@@ -127,7 +127,7 @@ BandArgs band_args(th_ctx* c, uint32_t off) {
 const uint64_t* pk_pairs(th_ctx* c, const th_pk* pk) {
   if (!pk->dp) {
     uint64_t* p = (uint64_t*)c->pool.get(2 * 2 * (size_t)c->L * c->N * 8);
-    HIPCHK(launch_prepare_pairs(pk->d, p, c->d_bc, c->d_lc, c->N, c->L, 2, c->stream));
+    HIPCHK(launch_prepare_pairs(pk->d, p, c->d_bc, c->d_lc.p, c->N, c->L, 2, c->stream));
     pk->dp = p;
   }
   return pk->dp;
@@ -181,10 +181,16 @@ void ntt_list(OpScope& sc, bool inverse, const std::vector<NttJob>& jobs, NttLoa
 }
 
 // ---------------------------------------------------------------- context setup
+static PmTw pm_tw(uint64_t w, uint64_t q) {
+  const uint64_t v = (uint64_t)(((u128)w << 32) % q), m30 = (1u << 30) - 1;
+  return PmTw{(uint32_t)(w & m30), (uint32_t)(w >> 30), (uint32_t)(v & m30), (uint32_t)(v >> 30)};
+}
+
 void build_tables(th_ctx* c) {
   const uint32_t N = c->N, L = c->L;
   std::vector<BarrettConst> bc(L);
   c->h_lc.resize(L);
+  c->d_lc.pm = std::all_of(c->q.begin(), c->q.end(), [](uint64_t q) { return q < FP64_PRIME_LIMIT || pm_prime(q); });
   // twiddles: per limb forward then inverse, N pairs of 16 bytes each; at the
   // split kernels' sizes followed by the row tables (row_table_index), per
   // limb forward then inverse, 15 N / 16 pairs each
@@ -208,12 +214,16 @@ void build_tables(th_ctx* c) {
       p = (uint64_t)(((u128)p * psi) % q);
       pi = (uint64_t)(((u128)pi * psi_inv) % q);
     }
-    const bool fp = q < FP64_PRIME_LIMIT;
+    const bool fp = q < FP64_PRIME_LIMIT, pm = c->d_lc.pm && !fp;
     unsigned char* fdst = host_tab.data() + (size_t)(2 * l) * N * 16;
     unsigned char* idst = host_tab.data() + (size_t)(2 * l + 1) * N * 16;
     for (uint32_t i = 0; i < N; ++i) {
       if (fp) {
         Fp64Tw a{(double)fw[i], (double)fw[i] / (double)q}, b{(double)iw[i], (double)iw[i] / (double)q};
+        memcpy(fdst + 16 * (size_t)i, &a, 16);
+        memcpy(idst + 16 * (size_t)i, &b, 16);
+      } else if (pm) {
+        const PmTw a = pm_tw(fw[i], q), b = pm_tw(iw[i], q);
         memcpy(fdst + 16 * (size_t)i, &a, 16);
         memcpy(idst + 16 * (size_t)i, &b, 16);
       } else {
@@ -253,16 +263,22 @@ void build_tables(th_ctx* c) {
     lc.inv = (const char*)c->d_tables + (size_t)(2 * l + 1) * N * 16;
     lc.fwd_row = split ? (const char*)c->d_tables + main_bytes + (size_t)(2 * l) * row_n * 16 : nullptr;
     lc.inv_row = split ? (const char*)c->d_tables + main_bytes + (size_t)(2 * l + 1) * row_n * 16 : nullptr;
-    lc.fp64 = fp ? 1 : 0;
+    lc.kind = fp ? LIMB_FP64 : pm ? LIMB_PM : LIMB_INT;
+    if (pm) {
+      lc.pm_c = (uint32_t)((1ULL << 60) - q);
+      lc.pm_n_inv = pm_tw(lc.n_inv, q);
+      lc.pm_last = pm_tw(lc.last_w, q);
+    }
     const u128 r = (~(u128)0) / q;
     uint64_t qi = 1;  // q^{-1} mod 2^64 by Newton's iteration (each step doubles the correct bits)
     for (int it = 0; it < 6; ++it) qi *= 2 - q * qi;
     const uint64_t r64 = (uint64_t)(((u128)1 << 64) % q);
-    bc[l] = BarrettConst{q, (uint64_t)(r >> 64), (uint64_t)r, (uint64_t)0 - qi, r64, (uint64_t)(((u128)r64 << 64) / q)};
+    bc[l] = BarrettConst{q, (uint64_t)(r >> 64), (uint64_t)r, (uint64_t)0 - qi, r64, (uint64_t)(((u128)r64 << 64) / q),
+                         lc.pm_c};
   }
   HIPCHK(hipMemcpy(c->d_tables, host_tab.data(), tab_bytes, hipMemcpyHostToDevice));
-  HIPCHK(hipMalloc(&c->d_lc, L * sizeof(LimbConst)));
-  HIPCHK(hipMemcpy(c->d_lc, c->h_lc.data(), L * sizeof(LimbConst), hipMemcpyHostToDevice));
+  HIPCHK(hipMalloc(&c->d_lc.p, L * sizeof(LimbConst)));
+  HIPCHK(hipMemcpy(c->d_lc.p, c->h_lc.data(), L * sizeof(LimbConst), hipMemcpyHostToDevice));
   HIPCHK(hipMalloc(&c->d_bc, L * sizeof(BarrettConst)));
   HIPCHK(hipMemcpy(c->d_bc, bc.data(), L * sizeof(BarrettConst), hipMemcpyHostToDevice));
   HIPCHK(hipMalloc(&c->d_q, L * 8));
@@ -285,6 +301,7 @@ void build_tables(th_ctx* c) {
       x.inv_dq = (double)x.inv / (double)q;  // correctly rounded: both operands are exact (q < 2^53)
       x.k32 = (double)((1ULL << 32) % q);
       x.k32q = x.k32 / (double)q;
+      if (c->h_lc[l].kind == LIMB_PM) x.pm_inv = pm_tw(x.inv, q);
     }
   }
   HIPCHK(hipMalloc(&c->d_rc, rc.size() * sizeof(RescaleConst)));
@@ -326,7 +343,7 @@ void destroy_ctx(th_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   c->pool.release_all();
   c->ring.destroy();
-  void* bufs[] = {c->d_lc, c->d_bc, c->d_q, c->d_rc, c->d_dc, c->d_twist_re, c->d_twist_im,
+  void* bufs[] = {c->d_lc.p, c->d_bc, c->d_q, c->d_rc, c->d_dc, c->d_twist_re, c->d_twist_im,
                   c->d_stage_re, c->d_stage_im, c->d_tables, c->bflag_gen, c->key_end};
   for (void* p : bufs)
     if (p) (void)hipFree(p);

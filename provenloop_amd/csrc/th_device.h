@@ -5,14 +5,21 @@
 // component L limb-polynomials back to back (the reference's RnsPoly layout,
 // tensafe-he-core/src/rns.rs:199-206, made contiguous).
 //
-// Two exact modular-multiply paths are used, chosen per prime:
+// Three exact modular-multiply paths are used, chosen per prime (LimbKind):
 //  * "int":  64-bit Shoup multiply with a precomputed floor(w*2^64/q) and
 //            Harvey-style lazy reduction; any q < 2^61.
 //  * "fp64": for q < 2^41 the product w*x is split exactly into hi + lo with
 //            one FMA and the quotient comes from x*(w/q) rounded to nearest;
 //            the remainder is exact (all intermediate integers < 2^53). Six
 //            full-rate FP64 instructions per multiply.
-// Both produce the unique canonical residue, so results are bit-identical to
+//  * "pm":   for q = 2^60 - c with a small c (the 60-bit primes of every
+//            default chain) 2^60 = c mod q, so a product is folded at bit 60
+//            instead of divided: no quotient is formed. 12 instructions per
+//            product by a fixed operand against the Shoup product's 14 and,
+//            since one fold takes any 64-bit value below q + 16 c, a forward
+//            butterfly of 16 instructions (one fold of half the values every
+//            four stages) against 22 with a conditional subtraction each.
+// All produce the unique canonical residue, so results are bit-identical to
 // the reference's u128 Barrett multiply (tensafe-he-core/src/rns.rs:45-95).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -23,6 +30,17 @@ namespace th {
 // Largest prime that takes the fp64 multiply path.
 constexpr uint64_t FP64_PRIME_LIMIT = 1ULL << 41;
 
+// A prime q takes the pm path when 2^60 - 2^26 < q < 2^60.
+constexpr uint64_t PM_MAX_C = 1ULL << 26;
+constexpr bool pm_prime(uint64_t q) { return q < (1ULL << 60) && q > (1ULL << 60) - PM_MAX_C; }
+enum LimbKind : uint32_t { LIMB_INT = 0, LIMB_FP64 = 1, LIMB_PM = 2 };
+
+// A fixed operand w < q of a pm product in 30-bit halves, w = wl + wh 2^30,
+// beside v = w 2^32 mod q likewise: x w = x0 w + x1 v (mod q) for the 32-bit
+// halves of x, and no sum of two partial products passes 2^63.
+struct PmTw {
+  uint32_t wl, wh, vl, vh;
+};
 struct ShoupTw {
   uint64_t w, ws;  // twiddle and floor(w * 2^64 / q)
 };
@@ -38,12 +56,23 @@ struct LimbConst {
   double qd, qinv;            // q and 1/q as doubles (fp64 path)
   double n_inv_d, n_inv_dq;
   double last_wd, last_wdq;
-  const void* fwd;            // N twiddle pairs (ShoupTw or Fp64Tw), fwd[brv(i)] = psi^i
+  PmTw pm_n_inv, pm_last;     // n_inv and last_w for the pm path
+  const void* fwd;            // N twiddle pairs (ShoupTw, Fp64Tw or PmTw), fwd[brv(i)] = psi^i
   const void* inv;            // N twiddle pairs, inv[brv(i)] = psi^-i
   const void* fwd_row;        // fwd and inv entries of the split row passes' lane-bit stages
   const void* inv_row;        //   in the order their lanes read them (row_table_index)
-  uint32_t fp64;              // 1 if this limb uses the fp64 path
-  uint32_t pad_;
+  uint32_t kind;              // LimbKind
+  uint32_t pm_c;              // 2^60 - q (pm path)
+};
+
+// A context's limb constants in device memory, and whether its chain takes the
+// pm path: every prime is a pm prime or below 2^41. Chains that mix in other
+// large primes take the int path for all of them, so each transform kernel
+// carries two arithmetics, fp64 and one of int and pm.
+struct LimbTable {
+  LimbConst* p = nullptr;
+  uint32_t pm = 0;
+  __device__ __forceinline__ const LimbConst& operator[](uint32_t l) const { return p[l]; }
 };
 
 // ---------------------------------------------------------------- int path
@@ -156,6 +185,7 @@ struct BarrettConst {
   uint64_t mq;          // -q^{-1} mod 2^64 (Montgomery products)
   uint64_t r64;         // 2^64 mod q (into Montgomery form)
   uint64_t r64_s;       // floor(r64 2^64 / q): its Shoup companion
+  uint64_t pm_c;        // 2^60 - q on the pm path, else 0
 };
 
 __device__ __forceinline__ uint64_t mulmod_barrett(uint64_t a, uint64_t b, const BarrettConst& m) {
@@ -197,6 +227,70 @@ __device__ __forceinline__ uint64_t submod(uint64_t a, uint64_t b, uint64_t q) {
   return a >= b ? a - b : a + q - b;
 }
 
+// ---------------------------------------------------------------- pm path
+// q = 2^60 - c, 0 < c < 2^26.
+//
+// x mod q, below q + 16 c, for any 64-bit x: the bits from 60 on fold to
+// multiples of c (three instructions).
+__device__ __forceinline__ uint64_t pm_fold(uint64_t x, uint32_t c) {
+  const uint32_t h = (uint32_t)(x >> 32);
+  return (uint64_t)(h >> 28) * c + (((uint64_t)(h & 0x0fffffffu) << 32) | (uint32_t)x);
+}
+// x mod q, canonical, for any 64-bit x.
+__device__ __forceinline__ uint64_t pm_canon(uint64_t x, uint64_t q, uint32_t c) {
+  return csub_n(pm_fold(x, c), q, opaque_u64(0 - q));
+}
+// x w mod q in [0, 2.5 q) for any 64-bit x. With ab = x0 wl + x1 vl and
+// cd = x0 wh + x1 vh (each at most 2^63 - 2^33 - 2^31 + 2: no overflow) the
+// product is ab + cd 2^30; its bits from 61 on, cd >> 31 (at most 2^32 - 5)
+// plus the at most 4 from the lower part's sum, are one 32-bit word h, and
+// h 2^61 = 2 h c. The result is below 2^61 + 2^32 2c <= 2^61 + 2^59.
+__device__ __forceinline__ uint64_t pm_mul_fixed(uint64_t x, const PmTw& t, uint32_t c2) {
+  const uint32_t x0 = (uint32_t)x, x1 = (uint32_t)(x >> 32);
+  const uint64_t ab = (uint64_t)x1 * t.vl + (uint64_t)x0 * t.wl;
+  const uint64_t cd = (uint64_t)x1 * t.vh + (uint64_t)x0 * t.wh;
+  const uint32_t top = __builtin_amdgcn_alignbit((uint32_t)(cd >> 32), (uint32_t)cd, 31);
+  const uint64_t d = ((uint64_t)((uint32_t)cd & 0x7fffffffu) << 30) + ab;
+  const uint32_t dh = (uint32_t)(d >> 32);
+  const uint32_t h = top + (dh >> 29);
+  return (uint64_t)h * c2 + (((uint64_t)(dh & 0x1fffffffu) << 32) | (uint32_t)d);
+}
+// a b mod q in [0, 4q) for a < 2^62, b < 2^60, neither with a companion: from
+// 30-bit halves a b = p11 2^60 + mid 2^30 + p00, and with mid = mh 2^30 + ml
+//   a b = (p11 + mh) c + ml 2^30 + p00  (mod q).
+// (p11 + mh) c has up to 88 bits: e0 c below, y = e1 c (< 2^57) times 2^32
+// above, whose bits from 28 on fold once more. Every term is below 2^60 + 2^58.
+__device__ __forceinline__ uint64_t pm_mul(uint64_t a, uint64_t b, uint32_t c) {
+  constexpr uint32_t M30 = (1u << 30) - 1, M28 = (1u << 28) - 1;
+  const uint32_t a0 = (uint32_t)a & M30, b0 = (uint32_t)b & M30;
+  const uint32_t a1 = __builtin_amdgcn_alignbit((uint32_t)(a >> 32), (uint32_t)a, 30);
+  const uint32_t b1 = __builtin_amdgcn_alignbit((uint32_t)(b >> 32), (uint32_t)b, 30);
+  const uint64_t p00 = (uint64_t)a0 * b0, mid = (uint64_t)a1 * b0 + (uint64_t)a0 * b1;
+  const uint64_t e = (uint64_t)a1 * b1 + (mid >> 30);
+  const uint32_t ml = (uint32_t)mid & M30;
+  const uint64_t r = ((uint64_t)ml << 30) + p00 + (uint64_t)(uint32_t)e * c;
+  const uint64_t y = (uint64_t)(uint32_t)(e >> 32) * c;
+  const uint32_t yh = __builtin_amdgcn_alignbit((uint32_t)(y >> 32), (uint32_t)y, 28);
+  return r + ((uint64_t)((uint32_t)y & M28) << 32) + (uint64_t)yh * c;
+}
+// A residue of e + 8c, below q + 16 c, for any signed e: e + 2^63 is unsigned,
+// and 2^63 = 8c (mod q).
+__device__ __forceinline__ uint64_t pm_fold_signed(int64_t e, uint32_t c) {
+  return pm_fold((uint64_t)e ^ (1ULL << 63), c);
+}
+
+// Operands fixed for many products are kept prepared for the limb's general
+// product: Montgomery form, except on the pm path, which takes them as they
+// are (launch_to_montgomery). a * prepared(b) mod q, a < 2^62: below 2q from
+// the Montgomery product, below 4q from the pm product.
+__device__ __forceinline__ uint64_t prepared_mul(uint64_t a, uint64_t b, const BarrettConst& m) {
+  return m.pm_c ? pm_mul(a, b, (uint32_t)m.pm_c) : mont_mul(a, b, m);
+}
+// a * b mod q, canonical, for canonical operands on any limb.
+__device__ __forceinline__ uint64_t mulmod(uint64_t a, uint64_t b, const BarrettConst& m) {
+  return m.pm_c ? pm_canon(pm_mul(a, b, (uint32_t)m.pm_c), m.q, (uint32_t)m.pm_c) : mulmod_barrett(a, b, m);
+}
+
 // Rescale constants of one output limb l (ciphertext.rs:497-522).
 struct RescaleConst {
   uint64_t q, inv, inv_s;  // q_l, (q_last mod q_l)^{-1} and its Shoup companion
@@ -204,6 +298,7 @@ struct RescaleConst {
   double qd, qinv;         // q_l and 1/q_l as doubles (limbs below 2^41)
   double inv_d, inv_dq;    // inv and inv / q_l as doubles (limbs below 2^41)
   double k32, k32q;        // 2^32 mod q_l and that / q_l as doubles (limbs below 2^41)
+  PmTw pm_inv;             // inv for the pm path
 };
 
 // ---------------------------------------------------------------- fp64 path

@@ -75,7 +75,7 @@ struct NttJob {
 };
 
 struct NttArgs {
-  const LimbConst* lc;
+  LimbTable lc;
   const NttJob* jobs;  // non-null: explicit job list
   const uint64_t* src;
   uint64_t* dst;
@@ -104,7 +104,7 @@ struct RescaleDecryptJob {
   double scale;         // the rescaled ciphertext's scale
 };
 struct RescaleDecryptArgs {
-  const LimbConst* lc;          // limb 0 is lc[0]
+  LimbTable lc;                 // limb 0 is lc[0]
   const BarrettConst* bc;       // limb 0
   const RescaleConst* rc;       // limb 0 at the products' level
   const uint64_t* skm;          // the secret key's limb 0 in Montgomery form
