@@ -222,14 +222,14 @@ struct LoadOp {
   // Values a load leaves for the transform: canonical on the Int and Fp64
   // limbs (MULM below 2q, DOTM below 3q), below 4q forward and 8q inverse on
   // pm limbs.
-  // signed_residue_dev with |e| in [q, 2^53) reduced by one exact FP64 step:
+  // signed_residue_dev with |e| in [q, 2^52) reduced by one exact FP64 step:
   // quot = rint(|e| / q) is within one of the true quotient, and the remainder
   // fma(-quot, q, |e|) is an exact integer in (-q, q)
   __device__ __forceinline__ uint64_t enc_residue(int64_t e) const {
     const uint64_t a = e >= 0 ? (uint64_t)e : (uint64_t)0 - (uint64_t)e;
     uint64_t r = a;
     if (a >= bc.q) {
-      if (a < (1ULL << 53)) {
+      if (a < (1ULL << 52)) {
         const double ad = u64_to_f64(a);
         double t = __fma_rn(-__builtin_rint(ad * qinv), qd, ad);
         t = t < 0.0 ? t + qd : t;
@@ -394,9 +394,9 @@ struct StoreOp {
   template <class A>
   __device__ __forceinline__ uint64_t apply_prep(const A& ar, typename A::V x, uint64_t cp) const {
     if constexpr (std::is_same_v<A, Fp64Arith> && NAUX > 0) {
-      const double y = reduce_f64(x, rc.qd, rc.qinv);  // canonical transform output
+      // (c - x) * inv with the output as it is: |x| < 16 q, |c - x| < 2^46
       const double c = __builtin_bit_cast(double, cp);
-      const double r = mulmod_f64(c - y, rc.inv_d, rc.inv_dq, rc.qd);  // (c - y) * inv, |c - y| < q
+      const double r = mulmod_f64(c - x, rc.inv_d, rc.inv_dq, rc.qd);
       return f64_to_u64(r < 0.0 ? r + rc.qd : r);
     } else if constexpr (std::is_same_v<A, PmArith> && NAUX > 0) {
       // cp < 4q, the folded output below 2q

@@ -299,8 +299,8 @@ void build_tables(th_ctx* c) {
       x.qinv = 1.0 / (double)q;
       x.inv_d = (double)x.inv;
       x.inv_dq = (double)x.inv / (double)q;  // correctly rounded: both operands are exact (q < 2^53)
-      x.k32 = (double)((1ULL << 32) % q);
-      x.k32q = x.k32 / (double)q;
+      x.q32 = (double)q * 0x1p-32;
+      x.r32 = 0x1p32 / (double)q;
       if (c->h_lc[l].kind == LIMB_PM) x.pm_inv = pm_tw(x.inv, q);
     }
   }

@@ -297,7 +297,7 @@ struct RescaleConst {
   BarrettConst b;          // remainder of a 64-bit value modulo q_l
   double qd, qinv;         // q_l and 1/q_l as doubles (limbs below 2^41)
   double inv_d, inv_dq;    // inv and inv / q_l as doubles (limbs below 2^41)
-  double k32, k32q;        // 2^32 mod q_l and that / q_l as doubles (limbs below 2^41)
+  double q32, r32;         // q_l / 2^32 (exact) and 2^32 / q_l (limbs below 2^41)
   PmTw pm_inv;             // inv for the pm path
 };
 
@@ -311,27 +311,29 @@ __device__ __forceinline__ double mulmod_f64(double x, double w, double wq, doub
   return r + lo;
 }
 
-// c mod q_l for any c < 2^61 on a limb below 2^41, as an exact double in
-// [0, q_l): with c = ch 2^32 + cl (ch < 2^29), c = ch (2^32 mod q_l) + cl
-// (mod q_l), the first term an exact FP64 product in (-q_l, q_l) and cl < q_l.
+// A residue of any c < 2^61 modulo a limb q_l below 2^41, as an exact double
+// below 0.52 q_l + 2^32 in magnitude, the forward transforms' input: with c =
+// ch 2^32 + cl (ch < 2^29) and quot = rint(ch 2^32 / q_l), ch - quot q_l / 2^32
+// is an exact multiple of 2^-32 (one FMA), and times 2^32 plus cl the residue
+// (another). Six instructions; through 2^32 mod q_l and corrected into [0,
+// q_l) it took 17, a third of the rescale column kernel's instructions on
+// these limbs.
 __device__ __forceinline__ double reduce_u64_f64(uint64_t c, const RescaleConst& rc) {
   const double ch = (double)(uint32_t)(c >> 32), cl = (double)(uint32_t)c;
-  double r = mulmod_f64(ch, rc.k32, rc.k32q, rc.qd) + cl;  // (-q_l, 2 q_l)
-  r = r < 0.0 ? r + rc.qd : r;
-  return r >= rc.qd ? r - rc.qd : r;
+  const double quot = __builtin_rint(ch * rc.r32);
+  return __fma_rn(__fma_rn(-quot, rc.q32, ch), 0x1p32, cl);
 }
 
-// a*b mod q in [0, q) for integers 0 <= a, b < q < 2^41 held exactly in
-// doubles, without a precomputed companion: hi + lo = a*b exactly (one FMA),
-// and quot = rint(hi / q) through qinv = 1/q is within 0.5 + 2^-10 of a*b/q
-// (a*b/q < 2^41, relative error below 2^-51), so r = a*b - quot*q, formed
-// exactly, lies in (-q, q).
+// a*b mod q within 0.51 q of zero for integers 0 <= a, b < q < 2^41 held
+// exactly in doubles, without a precomputed companion: hi + lo = a*b exactly
+// (one FMA), and quot = rint(hi / q) through qinv = 1/q is within 0.5 + 2^-10
+// of a*b/q (a*b/q < 2^41, relative error below 2^-51), and a*b - quot*q is
+// formed exactly.
 __device__ __forceinline__ double mulmod_f64_any(double a, double b, double q, double qinv) {
   const double hi = a * b;
   const double lo = __fma_rn(a, b, -hi);
   const double quot = __builtin_rint(hi * qinv);
-  const double r = __fma_rn(-quot, q, hi) + lo;
-  return r < 0.0 ? r + q : r;
+  return __fma_rn(-quot, q, hi) + lo;
 }
 
 // x mod q into [0, q) for an exact integer |x| < 2^50.
@@ -347,7 +349,13 @@ __device__ __forceinline__ double reduce_f64_signed(double x, double q, double q
   return __fma_rn(-quot, q, x);
 }
 
-__device__ __forceinline__ double u64_to_f64(uint64_t x) { return (double)x; }  // exact for x < 2^53
-__device__ __forceinline__ uint64_t f64_to_u64(double x) { return (uint64_t)x; }  // x integral, 0 <= x < 2^53
+// Between integers 0 <= x < 2^52 and doubles through the bits of 2^52 + x: two
+// instructions each way (the general conversions take four and six).
+__device__ __forceinline__ double u64_to_f64(uint64_t x) {
+  return __builtin_bit_cast(double, x | 0x4330000000000000ULL) - 0x1p52;
+}
+__device__ __forceinline__ uint64_t f64_to_u64(double x) {
+  return __builtin_bit_cast(uint64_t, x + 0x1p52) & 0x000fffffffffffffULL;
+}
 
 }  // namespace th

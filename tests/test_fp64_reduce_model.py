@@ -1,8 +1,9 @@
-"""Exact model of the FP64 reduction the rescale's fused column kernel uses.
+"""Exact model of an FP64 reduction of a 61-bit value to its canonical residue.
 
-For a limb prime q below 2^41 the kernel reduces the coefficient-domain last
-limb c (any c < 2^61) modulo q without 64-bit multiplies (reduce_u64_f64 in
-provenloop_amd/csrc/th_device.h): with c = ch 2^32 + cl,
+For a limb prime q below 2^41 the rescale needs the coefficient-domain last
+limb c (any c < 2^61) modulo q without 64-bit multiplies. The kernel takes a
+form without corrections (test_fp64_lazy_model.py); this is the canonical one,
+built from the butterflies' product: with c = ch 2^32 + cl,
 
     r = mulmod_f64(ch, 2^32 mod q) + cl,   then r < 0 -> r + q, r >= q -> r - q
 
@@ -12,7 +13,7 @@ This model performs the same IEEE-754 double operations (products and sums
 rounded to nearest even by Python's floats, fused multiply-adds rounded once
 from the exact rational value, rint ties to even) and checks the result
 against c mod q, so a wrong constant, a dropped term or a missing correction
-fails here; the GPU parity tests check the kernel's output bit for bit.
+fails here; the GPU parity tests check the kernels' output bit for bit.
 """
 from fractions import Fraction
 
