@@ -34,6 +34,16 @@
 //     P1: col = (l mod 2^(CB-4)) | (k << (CB-4))              registers = col bits [CB-4, CB)
 //     P2: col = k | ((l mod 2^(CB-4)) << 4)                   registers = col bits [0, 4)
 //     G:  e = l + 64 k                                        (lane-contiguous global access)
+// Where an encryption's or a rescale's transforms exceed the memory-side cache
+// (stream_launch), their intermediate and the rescale's output are streamed: they are
+// written, and the intermediate read, once by a launch, so their accesses carry
+// the nontemporal hint and leave the caches to the twiddles, the ciphertexts
+// and the plaintexts that several workgroups read. Per 7B-shape session-token
+// (N = 32768, 3.3 GB of it): encrypt column pass 140 -> 106 us,
+// rescale column kernel 1159 -> 1108, fused-rescale row pass 1868 -> 1766.
+// Launches that fit keep plain accesses: with the hint on all of them a
+// CryptoMOE token went from 692 to 713 us, and the batched inverse at N = 32768
+// (hint on its passes) from 82 to 88-98.
 // Column-pass wavefronts 2m and 2m+1 share the 128-byte lines of the
 // natural layout; they are given workgroup ids that the dispatcher sends to
 // the same XCD (ids are dealt round-robin over the 8 XCDs), so the second
@@ -62,6 +72,27 @@ struct Split {
   static constexpr int TWI = ((1 << (CB - 4)) - 1) << (10 - CB);
   static_assert(CB >= 4 && RB >= 4 && RB <= 10 && CB <= 10, "unsupported split");
 };
+
+// (STREAM is a template parameter throughout: of a branch between an access with
+// the hint and the same one without, the compiler makes one without.)
+template <bool STREAM, class T>
+__device__ __forceinline__ void store_hint(T v, GMut<T> p) {
+  if constexpr (STREAM)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+// The 16 intermediate values at buf[at(k)].
+template <bool STREAM, class A, class At>
+__device__ __forceinline__ void load_raw(typename A::V (&x)[16], const A& ar, GPtr<uint64_t> buf, const At& at) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    if constexpr (STREAM)
+      x[k] = ar.unraw(__builtin_nontemporal_load(&buf[at(k)]));
+    else
+      x[k] = ar.unraw(buf[at(k)]);
+  }
+}
 
 __device__ __forceinline__ uint32_t pad16(uint32_t e) { return e + (e >> 4); }
 
@@ -244,7 +275,7 @@ struct ColumnMap {
 // Forward column pass on coefficients already in registers (Q1 layout, the
 // arithmetic's representation); writes the intermediate to dst (Q2). HALF:
 // the exchange goes through half the LDS (wave_exchange_half).
-template <int LOGN, class A, bool BATCH = false, bool HALF = false>
+template <int LOGN, class A, bool STREAM, bool BATCH = false, bool HALF = false>
 __device__ __forceinline__ void column_fwd_regs(typename A::V (&x)[16], uint64_t* dst, const LimbConst& lc,
                                                 const ColumnMap<LOGN>& m, const A& ar, uint64_t* lds_raw) {
   constexpr int CB = Split<LOGN>::CB;
@@ -257,7 +288,7 @@ __device__ __forceinline__ void column_fwd_regs(typename A::V (&x)[16], uint64_t
   exchange_in<HALF>(x, lds_raw, [&](uint32_t k) { return m.e1(k); }, [&](uint32_t k) { return m.e2(k); });
   fwd_stages<LOGN, CB, LOGN - 5, CB, A, BATCH>(x, m.j2(0), tw, ar);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) gdst[m.j2(k)] = ar.raw(x[k]);
+  for (int k = 0; k < 16; ++k) store_hint<STREAM>(ar.raw(x[k]), &gdst[m.j2(k)]);
 }
 
 // Inverse column pass from the row pass's intermediate in buf (Q2); leaves
@@ -280,7 +311,7 @@ __device__ __forceinline__ void column_inv_regs(typename A::V (&x)[16], const ui
       x, 0u, [&](int, uint32_t base, uint32_t s) { return ld16_uniform(tw, base | s); }, ar, lc);
 }
 
-template <int LOGN, bool INV, class A, class LOp>
+template <int LOGN, bool INV, bool STREAM, class A, class LOp>
 __device__ __forceinline__ void column_pass(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst,
                                             const LimbConst& lc, const LOp& op, uint32_t part, uint64_t* lds_raw) {
   const ColumnMap<LOGN> m(part);
@@ -298,7 +329,7 @@ __device__ __forceinline__ void column_pass(const uint64_t* __restrict__ src, ui
 #pragma unroll
       for (int k = 0; k < 16; ++k) x[k] = ar.load(op.template at<A>(src, m.j1(k)));
     }
-    column_fwd_regs<LOGN, A, false, true>(x, dst, lc, m, ar, lds_raw);
+    column_fwd_regs<LOGN, A, STREAM, false, true>(x, dst, lc, m, ar, lds_raw);
   } else {
     column_inv_regs<LOGN>(x, dst, lc, m, ar, lds_raw);
     const GMut<uint64_t> gdst = gst(dst);
@@ -343,7 +374,7 @@ struct RowStage {
 // leaves the transform's outputs (the arithmetic's representation) in
 // registers in the lane-contiguous layout G: x[k] is element part * 1024 +
 // lane + 64 k.
-template <int LOGN, class A>
+template <int LOGN, bool STREAM, class A>
 __device__ __forceinline__ void row_fwd_regs(typename A::V (&x)[16], const uint64_t* buf, const LimbConst& lc,
                                              const A& ar, uint32_t part, uint64_t* lds_raw) {
   constexpr int CB = Split<LOGN>::CB, M = (1 << (CB - 4)) - 1;
@@ -357,8 +388,7 @@ __device__ __forceinline__ void row_fwd_regs(typename A::V (&x)[16], const uint6
   const GPtr<uint64_t> gbuf = gld(buf);
   const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd));
   const GPtr<typename A::Tw> tr = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd_row));
-#pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = ar.unraw(gbuf[jbase + p1(k)]);
+  load_raw<STREAM>(x, ar, gbuf + jbase, p1);
   fwd_stages<LOGN, CB - 4, CB - 1, CB - 4>(x, jbase + p1(0), tw, ar);
   wave_exchange(x, lds, p1, p2);
   // the stages on the P2 register bits read the row table (one load of
@@ -369,7 +399,7 @@ __device__ __forceinline__ void row_fwd_regs(typename A::V (&x)[16], const uint6
   wave_exchange(x, lds, p2, g);
 }
 
-template <int LOGN, bool INV, class A, class LOp, class SOp>
+template <int LOGN, bool INV, bool STREAM, class A, class LOp, class SOp>
 __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst,
                                          const LimbConst& lc, const LOp& op, const SOp& so, uint32_t part,
                                          uint64_t* lds_raw) {
@@ -393,8 +423,7 @@ __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint6
   };
   if constexpr (!INV) {
     const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd));
-#pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = ar.unraw(gdst[jbase + p1(k)]);
+    load_raw<STREAM>(x, ar, (GPtr<uint64_t>)gdst + jbase, p1);
     if constexpr (SOp::NAUX > 0) {
       // The store's operands and outputs in pairs of adjacent positions per
       // lane: register k is position h(k) = 2 lane + (k & 1) + 128 (k >> 1)
@@ -440,7 +469,7 @@ __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint6
         U2 o;
         o.x = so.apply_prep(ar, x[k], c[k]);
         o.y = so.apply_prep(ar, x[k + 1], c[k + 1]);
-        d2[(jbase + h(k)) >> 1] = o;
+        store_hint<STREAM>(o, &d2[(jbase + h(k)) >> 1]);
       }
     } else {
       fwd_stages<LOGN, CB - 4, CB - 1, CB - 4, A, false>(x, jbase + p1(0), tw, ar);
@@ -509,7 +538,7 @@ __device__ __forceinline__ uint32_t column_part(uint32_t p) {
 // the transform's input applies the fused load operation and the forward
 // row pass the fused store operation; otherwise passes read and write the
 // destination only.
-template <class BIG, int LOGN, bool INV, bool COLUMN, uint32_t LD, uint32_t ST>
+template <class BIG, int LOGN, bool INV, bool COLUMN, uint32_t LD, uint32_t ST, bool STREAM = false>
 __global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
   using S = Split<LOGN>;
   // the forward row pass with a fused rescale store, and the inverse row pass
@@ -543,9 +572,9 @@ __global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
   const LimbConst& lc = a.lc[limb];
   with_arith<BIG>(lc, [&]<class A>() {
     if constexpr (COLUMN)
-      column_pass<LOGN, INV, A>(src, dst, lc, op, part, lds);
+      column_pass<LOGN, INV, STREAM, A>(src, dst, lc, op, part, lds);
     else
-      row_pass<LOGN, INV, A>(src, dst, lc, op, so, part, lds);
+      row_pass<LOGN, INV, STREAM, A>(src, dst, lc, op, so, part, lds);
   });
 }
 
@@ -562,8 +591,8 @@ __global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
 // forward passes (workgroup b: part b % PARTS of forward job b / PARTS), so
 // the launch takes one inverse and one forward pass instead of the inverse
 // and nf forward passes in turn.
-template <class BIG, int LOGN>
-__global__ __launch_bounds__(64) void rescale_column_kernel(NttArgs inv, NttArgs fwd, uint32_t nf, uint32_t fan) {
+template <class BIG, int LOGN, bool STREAM>
+__global__ __launch_bounds__(64, 3) void rescale_column_kernel(NttArgs inv, NttArgs fwd, uint32_t nf, uint32_t fan) {
   using S = Split<LOGN>;
   __shared__ uint64_t lds[S::LDS];
   const uint32_t unit = blockIdx.x / S::PARTS;  // inverse job, or forward job with fan
@@ -602,9 +631,16 @@ __global__ __launch_bounds__(64) void rescale_column_kernel(NttArgs inv, NttArgs
         else
           x[k] = c[k] < rc.q ? c[k] : mulmod_barrett(c[k], 1, rc.b);
       }
-      column_fwd_regs<LOGN, A, true>(x, fj.dst, lcf, m, ar, lds);
+      column_fwd_regs<LOGN, A, STREAM, true>(x, fj.dst, lcf, m, ar, lds);
     });
   }
+}
+
+// Whether a forward launch of njobs limb-polynomials streams its data past the
+// caches: more than the 256 MiB of the memory-side cache.
+template <int LOGN>
+static bool stream_launch(uint32_t njobs) {
+  return ((uint64_t)njobs * 8 << LOGN) > (256u << 20);
 }
 
 // Largest fanned-out rescale column launch: one round of that kernel's
@@ -614,6 +650,7 @@ constexpr uint32_t RESCALE_FAN_MAX_WAVES = 3072;
 template <class BIG, int LOGN>
 static hipError_t launch_rescale_t(const NttArgs& inv, uint32_t ninv, const NttArgs& fwd, uint32_t nf, hipStream_t s) {
   using S = Split<LOGN>;
+  const bool stream = stream_launch<LOGN>(ninv * nf);
   const dim3 block(64);
   const hipError_t e = with_ops<true>(inv.load, inv.store, [&]<uint32_t LD, uint32_t ST>() -> hipError_t {
     if constexpr (ST != NTT_STORE_NONE) return hipErrorInvalidValue;  // segment sums: whole kernel only
@@ -625,13 +662,22 @@ static hipError_t launch_rescale_t(const NttArgs& inv, uint32_t ninv, const NttA
   // a batch whose nf passes per inverse job would leave most SIMDs idle
   // fans them out (RESCALE_FAN_MAX_WAVES)
   const uint32_t fan = ninv * nf * S::PARTS <= RESCALE_FAN_MAX_WAVES ? 1u : 0u;
-  hipLaunchKernelGGL((rescale_column_kernel<BIG, LOGN>), dim3(ninv * S::PARTS * (fan ? nf : 1)), block, 0, s, inv, fwd, nf,
-                     fan);
+  const dim3 grid(ninv * S::PARTS * (fan ? nf : 1));
+  if (stream)
+    hipLaunchKernelGGL((rescale_column_kernel<BIG, LOGN, true>), grid, block, 0, s, inv, fwd, nf, fan);
+  else
+    hipLaunchKernelGGL((rescale_column_kernel<BIG, LOGN, false>), grid, block, 0, s, inv, fwd, nf, fan);
   const hipError_t e2 = hipGetLastError();
   if (e2 != hipSuccess) return e2;
   return with_ops<false>(fwd.load, fwd.store, [&]<uint32_t LD, uint32_t ST>() -> hipError_t {
-    hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, false, NTT_LOAD_NONE, ST>), dim3(ninv * nf * S::PARTS), block, 0,
-                       s, fwd);
+    const dim3 rows(ninv * nf * S::PARTS);
+    if constexpr (StoreOp<ST>::NAUX > 0) {
+      if (stream) {
+        hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, false, NTT_LOAD_NONE, ST, true>), rows, block, 0, s, fwd);
+        return hipGetLastError();
+      }
+    }
+    hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, false, NTT_LOAD_NONE, ST>), rows, block, 0, s, fwd);
     return hipGetLastError();
   });
 }
@@ -663,7 +709,7 @@ hipError_t launch_rescale_split(int logn, const NttArgs& inv, uint32_t ninv, con
 // in dot.mask the kernel stores D = c0 + c1 s instead (EncDot): M's and E1's
 // wavefronts each hand the other half of their outputs over through LDS and
 // form D on their own half.
-template <class BIG, int LOGN>
+template <class BIG, int LOGN, bool STREAM>
 __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint64_t* pkp, uint64_t* cts, uint32_t L,
                                                           uint32_t mask, EncDot dot) {
   using S = Split<LOGN>;
@@ -685,7 +731,7 @@ __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint6
   auto run = [&]<class A>() {
     const A ar(lc);
     typename A::V x[16];
-    row_fwd_regs<LOGN>(x, jb[job].dst, lc, ar, part, lds[wv]);
+    row_fwd_regs<LOGN, STREAM>(x, jb[job].dst, lc, ar, part, lds[wv]);
     // the key pairs are requested before the barrier, so their latency
     // overlaps U's hand-over
     ShoupTw kp[16];
@@ -761,10 +807,16 @@ static hipError_t launch_encrypt_t(const NttArgs& a, uint32_t ninputs, uint32_t 
                                    const uint64_t* pkp, uint64_t* cts, hipStream_t s) {
   using S = Split<LOGN>;
   const uint32_t nl = (uint32_t)__builtin_popcount(mask);
-  hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, true, NTT_LOAD_ENC, NTT_STORE_NONE>),
-                     dim3(ninputs * 3 * nl * S::PARTS), dim3(64), 0, s, a);
-  hipLaunchKernelGGL((encrypt_row_kernel<BIG, LOGN>), dim3(ninputs * nl * S::PARTS), dim3(192), 0, s, a, pkp, cts, L,
-                     mask, dot);
+  const dim3 columns(ninputs * 3 * nl * S::PARTS), rows(ninputs * nl * S::PARTS);
+  if (stream_launch<LOGN>(ninputs * 3 * nl)) {
+    hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, true, NTT_LOAD_ENC, NTT_STORE_NONE, true>), columns, dim3(64),
+                       0, s, a);
+    hipLaunchKernelGGL((encrypt_row_kernel<BIG, LOGN, true>), rows, dim3(192), 0, s, a, pkp, cts, L, mask, dot);
+  } else {
+    hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, true, NTT_LOAD_ENC, NTT_STORE_NONE>), columns, dim3(64), 0, s,
+                       a);
+    hipLaunchKernelGGL((encrypt_row_kernel<BIG, LOGN, false>), rows, dim3(192), 0, s, a, pkp, cts, L, mask, dot);
+  }
   return hipGetLastError();
 }
 
@@ -873,7 +925,7 @@ __global__ __launch_bounds__(64) void rd_column_kernel(NttArgs inv, const Rescal
     typename A::V x[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.load(c[k]);
-    column_fwd_regs<LOGN, A, true>(x, ij.dst, lc0, m, ar, lds);
+    column_fwd_regs<LOGN, A, false, true>(x, ij.dst, lc0, m, ar, lds);
   });
 }
 
@@ -899,7 +951,7 @@ __global__ __launch_bounds__(64) void rd_row_kernel(RescaleDecryptArgs a) {
     const A ar(lc);
     typename A::V x[16];
     typename A::V* lds = reinterpret_cast<typename A::V*>(lds_raw);
-    row_fwd_regs<LOGN>(x, jb.y, lc, ar, part, lds_raw);
+    row_fwd_regs<LOGN, false>(x, jb.y, lc, ar, part, lds_raw);
     {
       // D pt - NTT(r1) s at positions jbase + g(k)
       const GPtr<uint64_t> d = gld(jb.d), p = gld(jb.ptm), sk = gld(a.skm);

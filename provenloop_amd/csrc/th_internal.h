@@ -89,7 +89,7 @@ struct NttArgs {
   const uint64_t* key;        // secret key, L x N (DOT)
   const double* segw;         // segment weight pairs, N x 2 (SEGSUM)
   uint32_t cols;              // segments per job (SEGSUM)
-  uint32_t pad_;
+  uint32_t stream;            // forward split passes: nontemporal hints (set by the launchers)
 };
 
 // One product ct x pt of a LoRA set, rescaled and decrypted on limb 0 into
