@@ -33,14 +33,11 @@ __device__ __forceinline__ double u128_to_f64(uint64_t hi, uint64_t lo) {
   return ldexp((double)mant, 75 - lz);
 }
 
-// Decrypted coefficient j, centred (or CRT-combined and centred), as f64.
-__device__ __forceinline__ double coeff_centred(const DecodeJob& jb, const DecodeConst& dc, uint32_t j, uint32_t n) {
-  if (!jb.crt) {
-    const uint64_t c = gld(jb.m)[j];
-    return c > dc.half_q0 ? -((double)(dc.q0 - c)) : (double)c;
-  }
+// A decrypted coefficient, centred (or CRT-combined and centred), as f64, from
+// its residues m0 mod q0 and (crt) m1 mod q1.
+__device__ __forceinline__ double centred(uint64_t m0, uint64_t m1, bool crt, const DecodeConst& dc) {
+  if (!crt) return m0 > dc.half_q0 ? -((double)(dc.q0 - m0)) : (double)m0;
   // ciphertext.rs:360-392
-  const uint64_t m0 = gld(jb.m)[j], m1 = gld(jb.m)[n + j];
   const uint64_t m0q1 = m0 < dc.q1 ? m0 : mulmod_barrett(m0, 1, dc.b1);
   const uint64_t diff = m1 >= m0q1 ? m1 - m0q1 : dc.q1 - m0q1 + m1;
   const uint64_t k = csub(shoup_lazy(diff, dc.q0_inv_q1, dc.q0_inv_q1_s, dc.q1), dc.q1);
@@ -62,14 +59,22 @@ __device__ __forceinline__ double coeff_centred(const DecodeJob& jb, const Decod
   return u128_to_f64(hi, lo);
 }
 
-// The reference's f64 coefficient value before the twist (encoding.rs:221-233,
-// ciphertext.rs:360-392): centred value / scale.
-__device__ __forceinline__ double coeff_value(const DecodeJob& jb, const DecodeConst& dc, uint32_t j, uint32_t n) {
-  return coeff_centred(jb, dc, j, n) / jb.scale;
+__device__ __forceinline__ double coeff_centred(const DecodeJob& jb, const DecodeConst& dc, uint32_t j, uint32_t n) {
+  return centred(gld(jb.m)[j], jb.crt ? gld(jb.m)[n + j] : 0, jb.crt, dc);
 }
 
 constexpr int DEC_THREADS = 1024;
+// Parts are added while a batch makes fewer workgroups than CUs: 112 decodes
+// at N = 16384 (the batched operations of 28 inputs) took 638 us a pass with
+// 256, 676 with 128 and 691 with the encoder's 512.
+constexpr uint32_t DEC_FILL = 256;
 
+// The in-part stages of part blockIdx.x of job blockIdx.y, over the elements
+// whose bit-reversed position lies in the part: the coefficient's f64 value
+// before the twist is centred value / scale (encoding.rs:221-233,
+// ciphertext.rs:360-392). A thread's 8 residues are requested together. One
+// decode cut into 16 parts of 1024 values takes 17 us where two parts of 8192,
+// on two of the 256 CUs, took 33 us (N = 16384).
 template <int LP>
 __global__ __launch_bounds__(DEC_THREADS) void k_decode_parts(const DecodeJob* __restrict__ jobs, const DecodeConst* dcp,
                                                               const double* __restrict__ twist_re,
@@ -79,29 +84,78 @@ __global__ __launch_bounds__(DEC_THREADS) void k_decode_parts(const DecodeJob* _
   extern __shared__ double sh[];
   const DecodeConst dc = *dcp;
   const uint32_t n = 1u << logn;
-  const uint32_t M = n >> LP;
+  const uint32_t M = n >> LP, MP = fft_pad(M);
   const uint32_t part = blockIdx.x;
   const DecodeJob jb = jobs[blockIdx.y];
   double* re = sh;
-  double* im = sh + M;
+  double* im = sh + MP;
   const uint32_t r = brv_bits(part, LP);
   const uint32_t lb = logn - LP;
-  for (uint32_t jj = threadIdx.x; jj < M; jj += blockDim.x) {
-    const uint32_t j = (jj << LP) | r;
-    const double c = coeff_value(jb, dc, j, n);
-    const uint32_t pos = brv_bits(jj, lb);
-    re[pos] = c * twist_re[j];
-    im[pos] = -c * twist_im[j];
+  const double *twr, *twi;
+  fft_stage_twiddles<LP>(sh + 2 * MP, M, stage_re, stage_im, twr, twi);
+  const GPtr<uint64_t> m = gld(jb.m);
+  for (uint32_t j0 = threadIdx.x; j0 < M; j0 += FFT_ROUND * blockDim.x) {
+    uint64_t m0[FFT_ROUND], m1[FFT_ROUND];
+    double tr[FFT_ROUND], ti[FFT_ROUND];
+#pragma unroll
+    for (int e = 0; e < FFT_ROUND; ++e) {
+      const uint32_t jj = j0 + e * blockDim.x;
+      const uint32_t j = ((jj < M ? jj : 0) << LP) | r;
+      m0[e] = m[j];
+      m1[e] = jb.crt ? m[n + j] : 0;
+      tr[e] = gld(twist_re)[j];
+      ti[e] = gld(twist_im)[j];
+    }
+#pragma unroll
+    for (int e = 0; e < FFT_ROUND; ++e) {
+      const uint32_t jj = j0 + e * blockDim.x;
+      if (jj >= M) break;
+      const double c = centred(m0[e], m1[e], jb.crt, dc) / jb.scale;
+      const uint32_t pos = fft_pad(brv_bits(jj, lb));
+      re[pos] = c * tr[e];
+      im[pos] = -c * ti[e];
+    }
   }
   __syncthreads();
-  dit_stages_reg(re, im, lb, stage_re, stage_im);
-  const GMut<double> out = gst(jb.parts) + (size_t)part * 2 * M;
-  for (uint32_t i = threadIdx.x; i < M; i += blockDim.x) {
-    out[i] = re[i];
-    out[M + i] = im[i];
+  dit_stages_reg<true>(re, im, lb, twr, twi);
+  fft_store_part(re, im, M, gst(jb.parts) + (size_t)part * 2 * M);
+}
+
+// The last LP stages and the slots (the real parts of the first N/2 outputs):
+// G threads share a position k, thread o of them writing the outputs at parts
+// s G + o of the first half; the operands and twiddles are those of one
+// transform of N values (combine_parts).
+template <int LP>
+__global__ __launch_bounds__(256) void k_decode_slots(const DecodeJob* __restrict__ jobs,
+                                                      const double* __restrict__ stage_re,
+                                                      const double* __restrict__ stage_im, uint32_t logn) {
+  constexpr int P = 1 << LP;
+  constexpr int G = P >= 4 ? P / 4 : 1;
+  const uint32_t M = (1u << logn) >> LP, lb = logn - LP;
+  const DecodeJob jb = jobs[blockIdx.y];
+  const GMut<double> out = gst(jb.out);
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < G * M; i += gridDim.x * blockDim.x) {
+    const uint32_t o = i >> lb, k = i & (M - 1);  // o is uniform over a wavefront (M >= 64)
+    Cx x[P];
+    combine_parts<LP>(gld(jb.parts), k, M, gld(stage_re), gld(stage_im), x);
+    if constexpr (LP == 0) {
+      if (k < M / 2) out[k] = x[0].re;
+    } else {
+#pragma unroll
+      for (int s = 0; s < P / 2 / G; ++s) {
+        double v = x[s * G].re;
+#pragma unroll
+        for (int g = 1; g < G; ++g)
+          if (o == (uint32_t)g) v = x[s * G + g].re;
+        out[(size_t)(s * G + o) * M + k] = v;
+      }
+    }
   }
 }
 
+// The last LP stages with the slots summed into segments in the same workgroup
+// (and the slots written where wanted): sums of more segments than the
+// segment-sum kernels take.
 template <int LP>
 __global__ __launch_bounds__(DEC_THREADS) void k_decode_final(const DecodeJob* __restrict__ jobs,
                                                               const double* __restrict__ stage_re,
@@ -229,9 +283,33 @@ hipError_t launch_decode(const DecodeJob* jobs, uint32_t njobs, const DecodeCons
                          const double* twist_im, const double* stage_re, const double* stage_im, uint32_t logn,
                          uint32_t d, uint32_t cols, hipStream_t s) {
   if (!njobs) return hipSuccess;
+  if (cols == 0) {  // slots only
+    const uint32_t lp = fft_batch_parts_log(logn, njobs, DEC_FILL), M = (1u << logn) >> lp;
+    const uint32_t threads = M / 8 < 64 ? 64 : (M / 8 > DEC_THREADS ? DEC_THREADS : M / 8);
+    const uint32_t fin = lp >= 2 ? M << (lp - 2) : M;
+    const size_t lds = fft_part_lds(logn, lp);
+#define TH_SLOTS(LP)                                                                                             \
+  case LP: {                                                                                                     \
+    const hipError_t e = allow_full_lds<k_decode_parts<LP>>();                                                   \
+    if (e != hipSuccess) return e;                                                                               \
+    hipLaunchKernelGGL(k_decode_parts<LP>, dim3(1u << LP, njobs), dim3(threads), lds, s, jobs, dc, twist_re,     \
+                       twist_im, stage_re, stage_im, logn);                                                      \
+    hipLaunchKernelGGL(k_decode_slots<LP>, dim3((fin + 255) / 256, njobs), dim3(256), 0, s, jobs, stage_re,      \
+                       stage_im, logn);                                                                          \
+    return hipGetLastError();                                                                                    \
+  }
+    switch (lp) {
+      TH_SLOTS(0)
+      TH_SLOTS(1)
+      TH_SLOTS(2)
+      TH_SLOTS(3)
+      TH_SLOTS(4)
+      default: return hipErrorInvalidValue;
+    }
+#undef TH_SLOTS
+  }
   const uint32_t lp = fft_parts_log(logn);
-  const uint32_t M = (1u << logn) >> lp;
-  const size_t lds_a = (size_t)2 * M * sizeof(double);
+  const size_t lds_a = fft_part_lds(logn, lp);
   const size_t lds_b = (size_t)(1u << logn) / 2 * sizeof(double);
   hipError_t e;
 #define TH_DEC(LP)                                                                                         \

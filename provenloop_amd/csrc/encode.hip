@@ -36,39 +36,9 @@ __device__ __forceinline__ void encode_part(const EncodeJob* __restrict__ jobs, 
   double* im = sh + MP;
   const uint32_t r = brv_bits(part, LP);
   const uint32_t lb = logn - LP;
-  // With 8 or more parts the in-part stages' twiddles (entries 0 .. M-2 of
-  // the stage tables) are staged in LDS beside the values, read in the same
-  // coalesced phase as the input instead of once per register pass.
-  constexpr bool TWL = LP >= 3;
-  const double* twr = stage_re;
-  const double* twi = stage_im;
-  // 8 entries of each table per thread per round (one round with
-  // blockDim.x = M / 8), all loads issued before the first LDS store
-  constexpr int FV = 8;
-  if constexpr (TWL) {
-    double* tr = sh + 2 * MP;
-    double* ti = sh + 2 * MP + M;
-    for (uint32_t i0 = threadIdx.x; i0 + 1 < M; i0 += FV * blockDim.x) {
-      double a[FV], b[FV];
-#pragma unroll
-      for (int e = 0; e < FV; ++e) {
-        const uint32_t i = i0 + e * blockDim.x;
-        const uint32_t ic = i + 1 < M ? i : 0;
-        a[e] = gld(stage_re)[ic];
-        b[e] = gld(stage_im)[ic];
-      }
-#pragma unroll
-      for (int e = 0; e < FV; ++e) {
-        const uint32_t i = i0 + e * blockDim.x;
-        if (i + 1 < M) {
-          tr[i] = a[e];
-          ti[i] = b[e];
-        }
-      }
-    }
-    twr = tr;
-    twi = ti;
-  }
+  const double *twr, *twi;
+  fft_stage_twiddles<LP>(sh + 2 * MP, M, stage_re, stage_im, twr, twi);
+  constexpr int FV = FFT_ROUND;
   // input gather, 8 values per thread per round: all loads issued before the
   // first LDS store
   const double g = jb.gate ? *gld(jb.gate) : 1.0;
@@ -102,25 +72,7 @@ __device__ __forceinline__ void encode_part(const EncodeJob* __restrict__ jobs, 
   }
   __syncthreads();
   dit_stages_reg<true>(re, im, lb, twr, twi);
-  const GMut<double> out = gst(jb.parts) + (size_t)part * 2 * M;
-  for (uint32_t i0 = threadIdx.x; i0 < M; i0 += FV * blockDim.x) {
-    double a[FV], b[FV];
-#pragma unroll
-    for (int e = 0; e < FV; ++e) {
-      const uint32_t i = i0 + e * blockDim.x;
-      const uint32_t ic = fft_pad(i < M ? i : 0);
-      a[e] = re[ic];
-      b[e] = im[ic];
-    }
-#pragma unroll
-    for (int e = 0; e < FV; ++e) {
-      const uint32_t i = i0 + e * blockDim.x;
-      if (i < M) {
-        out[i] = a[e];
-        out[M + i] = b[e];
-      }
-    }
-  }
+  fft_store_part(re, im, M, gst(jb.parts) + (size_t)part * 2 * M);
 }
 
 template <int LP>
@@ -195,25 +147,6 @@ __device__ __forceinline__ void emit_coefficient(const EncodeJob& jb, const Barr
     dst[(size_t)l * n + j] = jb.e0 ? csub(mm + signed_residue_dev(e0, c), c.q) : mm;
     if (jb.e1) dst[(size_t)(L + l) * n + j] = signed_residue_dev(e1, c);
     if (jb.u) dst[(size_t)(2 * L + l) * n + j] = u == 0 ? c.q - 1 : (u == 1 ? 0 : 1);
-  }
-}
-
-// The FFT outputs at positions p*M + k of all P parts (x[p]), from the parts' stage-lb values.
-template <int LP>
-__device__ __forceinline__ void combine_parts(GPtr<double> Pd, uint32_t k, uint32_t M, GPtr<double> wr,
-                                              GPtr<double> wi, Cx (&x)[1 << LP]) {
-  constexpr int P = 1 << LP;
-#pragma unroll
-  for (int p = 0; p < P; ++p) x[p] = Cx{Pd[(size_t)p * 2 * M + k], Pd[(size_t)p * 2 * M + M + k]};
-#pragma unroll
-  for (int t = 0; t < LP; ++t) {
-    const uint32_t half = M << t;
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      if (p & (1 << t)) continue;
-      const uint32_t w = half - 1 + (uint32_t)(p & ((1 << t) - 1)) * M + k;
-      dit(x[p], x[p | (1 << t)], wr[w], wi[w], x[p], x[p | (1 << t)]);
-    }
   }
 }
 
@@ -343,18 +276,12 @@ hipError_t launch_encode(const EncodeJob* jobs, uint32_t njobs, const BarrettCon
   if (sample && seeds)
     for (uint32_t i = 0; i < njobs; ++i) sb.v[i] = seeds[i];
   const int use_sb = seeds != nullptr;
-  // parts of at most 4096 values (two workgroups' LDS per CU; with 672
-  // encodes of N=16384 per CryptoMOE token, the token measured 0.656 ms with
-  // 4096-value parts against 0.697 ms with 8192, 0.675 ms with 2048 and
-  // 0.727 ms with 1024); more parts (up to 16, of at least 1024 values)
-  // while the batch would leave CUs idle: the parts are independent
-  // workgroups and the result is the same for any split
-  const uint32_t lp_min = fft_parts_log(logn);
-  uint32_t lp = logn > 12 && logn - 12 > lp_min ? logn - 12 : lp_min;
-  while (lp < 4 && logn - lp > 10 && njobs * (1u << lp) < 512) ++lp;
+  // 672 encodes of N=16384 per CryptoMOE token: the token measured 0.656 ms
+  // with parts of 4096 values against 0.697 ms with 8192, 0.675 ms with 2048
+  // and 0.727 ms with 1024
+  const uint32_t lp = fft_batch_parts_log(logn, njobs, 512);
   const uint32_t M = n >> lp;
-  // padded values (+ twiddles with 8 or more parts)
-  const size_t lds = ((size_t)2 * fft_pad(M) + (lp >= 3 ? (size_t)2 * M : 0)) * sizeof(double);
+  const size_t lds = fft_part_lds(logn, lp);
   // dit_stages_reg needs 8 values per thread at most
   const uint32_t threads = M / 8 < 64 ? 64 : (M / 8 > ENC_THREADS ? ENC_THREADS : M / 8);
   const uint32_t fin = lp >= 2 ? M << (lp - 2) : M;  // threads of the final kernel per encode

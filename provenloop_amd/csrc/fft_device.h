@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "th_device.h"
+
 namespace th {
 
 __device__ __forceinline__ uint32_t brv_bits(uint32_t x, uint32_t bits) {
@@ -125,5 +127,102 @@ __device__ __forceinline__ void dit_stages_reg(double* re, double* im, uint32_t 
 
 // Parts per transform: one part fits LDS (2^13 complex = 128 KiB).
 __host__ __device__ constexpr uint32_t fft_parts_log(uint32_t logn) { return logn <= 13 ? 0 : logn - 13; }
+
+// Values a thread moves per round of the phases around the stages: all of a
+// round's loads are issued before its first LDS store.
+constexpr int FFT_ROUND = 8;
+
+// With 8 or more parts the in-part stages' twiddles (entries 0 .. M-2 of the
+// stage tables) are staged in LDS at `lds` (2 M doubles), read in the same
+// coalesced phase as the input instead of once per register pass; twr, twi:
+// where the stages read them.
+template <int LP>
+__device__ __forceinline__ void fft_stage_twiddles(double* lds, uint32_t M, const double* __restrict__ stage_re,
+                                                   const double* __restrict__ stage_im, const double*& twr,
+                                                   const double*& twi) {
+  twr = stage_re;
+  twi = stage_im;
+  if constexpr (LP >= 3) {
+    double* tr = lds;
+    double* ti = lds + M;
+    for (uint32_t i0 = threadIdx.x; i0 + 1 < M; i0 += FFT_ROUND * blockDim.x) {
+      double a[FFT_ROUND], b[FFT_ROUND];
+#pragma unroll
+      for (int e = 0; e < FFT_ROUND; ++e) {
+        const uint32_t i = i0 + e * blockDim.x;
+        const uint32_t ic = i + 1 < M ? i : 0;
+        a[e] = gld(stage_re)[ic];
+        b[e] = gld(stage_im)[ic];
+      }
+#pragma unroll
+      for (int e = 0; e < FFT_ROUND; ++e) {
+        const uint32_t i = i0 + e * blockDim.x;
+        if (i + 1 < M) {
+          tr[i] = a[e];
+          ti[i] = b[e];
+        }
+      }
+    }
+    twr = tr;
+    twi = ti;
+  }
+}
+
+// A part's M values from LDS (fft_pad) to its scratch, real then imaginary.
+__device__ __forceinline__ void fft_store_part(const double* re, const double* im, uint32_t M, GMut<double> out) {
+  for (uint32_t i0 = threadIdx.x; i0 < M; i0 += FFT_ROUND * blockDim.x) {
+    double a[FFT_ROUND], b[FFT_ROUND];
+#pragma unroll
+    for (int e = 0; e < FFT_ROUND; ++e) {
+      const uint32_t i = i0 + e * blockDim.x;
+      const uint32_t ic = fft_pad(i < M ? i : 0);
+      a[e] = re[ic];
+      b[e] = im[ic];
+    }
+#pragma unroll
+    for (int e = 0; e < FFT_ROUND; ++e) {
+      const uint32_t i = i0 + e * blockDim.x;
+      if (i < M) {
+        out[i] = a[e];
+        out[M + i] = b[e];
+      }
+    }
+  }
+}
+
+// The FFT outputs at positions p*M + k of all P parts (x[p]), from the parts' stage-lb values.
+template <int LP>
+__device__ __forceinline__ void combine_parts(GPtr<double> Pd, uint32_t k, uint32_t M, GPtr<double> wr,
+                                              GPtr<double> wi, Cx (&x)[1 << LP]) {
+  constexpr int P = 1 << LP;
+#pragma unroll
+  for (int p = 0; p < P; ++p) x[p] = Cx{Pd[(size_t)p * 2 * M + k], Pd[(size_t)p * 2 * M + M + k]};
+#pragma unroll
+  for (int t = 0; t < LP; ++t) {
+    const uint32_t half = M << t;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      if (p & (1 << t)) continue;
+      const uint32_t w = half - 1 + (uint32_t)(p & ((1 << t) - 1)) * M + k;
+      dit(x[p], x[p | (1 << t)], wr[w], wi[w], x[p], x[p | (1 << t)]);
+    }
+  }
+}
+
+// log2 of the parts a batch of njobs transforms is cut into: parts of at most
+// 4096 values (two workgroups' LDS per CU), and more of them (up to 16, of at
+// least 1024 values) while the batch makes fewer than `fill` workgroups. The
+// parts are independent workgroups and the result is the same for any split.
+inline uint32_t fft_batch_parts_log(uint32_t logn, uint32_t njobs, uint32_t fill) {
+  const uint32_t lp_min = fft_parts_log(logn);
+  uint32_t lp = logn > 12 && logn - 12 > lp_min ? logn - 12 : lp_min;
+  while (lp < 4 && logn - lp > 10 && njobs * (1u << lp) < fill) ++lp;
+  return lp;
+}
+// LDS of one part's workgroup: padded values, and twiddles with 8 or more parts.
+inline size_t fft_part_lds(uint32_t logn, uint32_t lp) {
+  const uint32_t M = (1u << logn) >> lp;
+  return ((size_t)2 * fft_pad(M) + (lp >= 3 ? (size_t)2 * M : 0)) * sizeof(double);
+}
 
 }  // namespace th

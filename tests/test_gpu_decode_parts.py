@@ -1,0 +1,36 @@
+"""Batched decoding at every split of its FFT, bit for bit against the oracle.
+
+The number of parts (1 to 16) follows the ring and the batch size; N and counts
+on both sides of each change, both decryption branches (limb 0, and limbs 0 and
+1 combined where the scale exceeds 1.5 x 2^40).
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from provenloop_amd import tensafe_he
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,count", [(1024, 1), (1024, 3), (2048, 1), (4096, 2), (8192, 1), (8192, 33), (8192, 70),
+                                     (16384, 1), (16384, 33), (16384, 65), (16384, 130), (32768, 1), (32768, 33)])
+def test_batch_decrypt_matches_oracle(n, count):
+    q = orc.default_chain(max(n, 8192))
+    eng, ref = tensafe_he.CkksContext(n, moduli=q), orc.Context(n, moduli=q)
+    sk, rsk = eng.keygen(seed=5), ref.keygen(5)
+    pk, rpk = eng.keygen_public(sk, seed=6), ref.keygen_public(rsk, 6)
+    rng = np.random.default_rng(n + count)
+    v, w = rng.standard_normal(n // 2), rng.standard_normal(n // 2)
+    ct, rct = eng.encrypt_pk(v, pk, seed=7), ref.encrypt_pk(v, rpk, 7)
+    prod, rprod = ct * w, ref.ct_pt_mul(rct, w)
+    exp = [ref.decrypt(rct, rsk), ref.decrypt(rprod, rsk)]
+    cts = [(ct, prod)[i & 1] for i in range(count)]
+    dev = torch.empty((count, n // 2), dtype=torch.float64, device="cuda")
+    eng.batch_decrypt_to_device(cts, sk, dev.data_ptr())
+    eng.sync()
+    got = dev.cpu().numpy()
+    for i in range(count):
+        assert np.array_equal(got[i], exp[i & 1]), i
+    assert np.array_equal(eng.decrypt(prod, sk), exp[1])
