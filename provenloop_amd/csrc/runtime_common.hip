@@ -274,7 +274,7 @@ void build_tables(th_ctx* c) {
     for (int it = 0; it < 6; ++it) qi *= 2 - q * qi;
     const uint64_t r64 = (uint64_t)(((u128)1 << 64) % q);
     bc[l] = BarrettConst{q, (uint64_t)(r >> 64), (uint64_t)r, (uint64_t)0 - qi, r64, (uint64_t)(((u128)r64 << 64) / q),
-                         lc.pm_c};
+                         lc.pm_c, fp ? lc.qd : 0.0, fp ? lc.qinv : 0.0};
   }
   HIPCHK(hipMemcpy(c->d_tables, host_tab.data(), tab_bytes, hipMemcpyHostToDevice));
   HIPCHK(hipMalloc(&c->d_lc.p, L * sizeof(LimbConst)));
