@@ -64,6 +64,7 @@ int th_ctx_create(uint32_t N, const uint64_t* moduli, uint32_t L, uint32_t scale
       HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
       build_tables(c);
       c->ring.init(64u << 20);
+      c->slots.init();
       c->bflag_cap = 1u << 16;
       HIPCHK(hipHostMalloc((void**)&c->bflag_host, c->bflag_cap, hipHostMallocMapped | hipHostMallocCoherent));
       HIPCHK(hipHostGetDevicePointer((void**)&c->bflag_dev, c->bflag_host, 0));

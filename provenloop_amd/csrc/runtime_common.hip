@@ -343,6 +343,7 @@ void destroy_ctx(th_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   c->pool.release_all();
   c->ring.destroy();
+  c->slots.destroy();
   void* bufs[] = {c->d_lc.p, c->d_bc, c->d_q, c->d_rc, c->d_dc, c->d_twist_re, c->d_twist_im,
                   c->d_stage_re, c->d_stage_im, c->d_tables, c->bflag_gen, c->key_end};
   for (void* p : bufs)
