@@ -168,6 +168,10 @@ int th_encrypt_pk_batch(th_ctx* ctx, const th_pk* pk, const double* z, size_t n,
     need(z != nullptr || count == 0, "null input");
     if (!count) return;
     const size_t S = ctx->N / 2;
+    if (n >= S && stride == S) {  // whole rows back to back: nothing to pad
+      encrypt_pk_seeded(ctx, pk, z, count, seeds, outs);
+      return;
+    }
     std::vector<double> pad(count * S);
     for (size_t i = 0; i < count; ++i) pad_input(ctx, z + i * stride, n, pad.data() + i * S);
     encrypt_pk_seeded(ctx, pk, pad.data(), count, seeds, outs);

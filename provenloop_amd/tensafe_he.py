@@ -28,6 +28,11 @@ __all__ = ["CkksContext", "TenSafeCiphertext", "TenSafeSecretKey", "TenSafePubli
 
 _VERSION = "0.1.0"
 
+# PyBytes_FromStringAndSize(NULL, n): a bytes object to be filled in place
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype = C.py_object
+_new_bytes.argtypes = [C.c_char_p, C.c_ssize_t]
+
 
 def _as_f64_vector(data, what="data") -> np.ndarray:
     """PyReadonlyArray1<f64> + as_slice() semantics (lib.rs:119-123)."""
@@ -214,7 +219,7 @@ class CkksContext:
                          z.size, s, has)
 
     def decrypt(self, ct: TenSafeCiphertext, sk: TenSafeSecretKey) -> np.ndarray:
-        out = np.zeros(self.num_slots, np.float64)
+        out = np.empty(self.num_slots, np.float64)
         _lib.check(_lib.load().th_decrypt(self._h, self._own(ct), self._own(sk), _lib.ptr(out)))
         return out
 
@@ -286,10 +291,11 @@ class CkksContext:
         if not arrays:
             return []
         S = self.num_slots
-        flat = np.zeros((len(arrays), S), np.float64)
+        flat = np.empty((len(arrays), S), np.float64)
         for i, a in enumerate(arrays):
             z = self._pad(a, "arrays")
             flat[i, : z.size] = z
+            flat[i, z.size :] = 0.0
         sd = np.ascontiguousarray(seeds, dtype=np.uint64)
         outs = (C.c_void_p * len(arrays))()
         _lib.check(_lib.load().th_encrypt_pk_batch(self._h, self._own(pk), _lib.ptr(flat), S, S, len(arrays),
@@ -380,8 +386,8 @@ class CkksContext:
     # ------------------------------------------------------------ data movement (tests, wire format)
     def ct_download(self, ct: TenSafeCiphertext):
         limbs = ct.num_limbs
-        c0 = np.zeros((limbs, self._n), np.uint64)
-        c1 = np.zeros((limbs, self._n), np.uint64)
+        c0 = np.empty((limbs, self._n), np.uint64)
+        c1 = np.empty((limbs, self._n), np.uint64)
         _lib.check(_lib.load().th_ct_download(self._h, self._own(ct), _lib.ptr(c0), _lib.ptr(c1)))
         return c0, c1
 
@@ -394,18 +400,18 @@ class CkksContext:
                          c0.shape[0], float(scale))
 
     def sk_download(self, sk: TenSafeSecretKey) -> np.ndarray:
-        out = np.zeros((self._limbs, self._n), np.uint64)
+        out = np.empty((self._limbs, self._n), np.uint64)
         _lib.check(_lib.load().th_sk_download(self._h, self._own(sk), _lib.ptr(out)))
         return out
 
     def pk_download(self, pk: TenSafePublicKey):
-        b = np.zeros((self._limbs, self._n), np.uint64)
-        a = np.zeros((self._limbs, self._n), np.uint64)
+        b = np.empty((self._limbs, self._n), np.uint64)
+        a = np.empty((self._limbs, self._n), np.uint64)
         _lib.check(_lib.load().th_pk_download(self._h, self._own(pk), _lib.ptr(b), _lib.ptr(a)))
         return b, a
 
     def pt_download(self, pt: TenSafePlaintext) -> np.ndarray:
-        out = np.zeros((self._limbs, self._n), np.uint64)
+        out = np.empty((self._limbs, self._n), np.uint64)
         _lib.check(_lib.load().th_pt_download(self._h, self._own(pt), _lib.ptr(out)))
         return out
 
@@ -413,9 +419,10 @@ class CkksContext:
         n = C.c_size_t()
         f = getattr(_lib.load(), fn)
         _lib.check(f(self._h, self._own(obj), None, 0, C.byref(n)))
-        buf = np.zeros(n.value, np.uint8)
-        _lib.check(f(self._h, self._own(obj), _lib.ptr(buf), buf.size, C.byref(n)))
-        return buf.tobytes()
+        # the bytes object itself is the buffer: written once, before anything else sees it
+        out = _new_bytes(None, n.value)
+        _lib.check(f(self._h, self._own(obj), C.cast(C.c_char_p(out), C.c_void_p), n.value, C.byref(n)))
+        return out
 
     def ct_from_bytes(self, data: bytes, num_limbs: Optional[int] = None) -> TenSafeCiphertext:
         """serialize.rs:80-93 (num_limbs defaults to the context's chain length)."""
