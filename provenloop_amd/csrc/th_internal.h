@@ -22,8 +22,9 @@ namespace th {
 //            0: x = (m + e0) mod q, src = m, aux = e0 (i64 coefficients)
 //            1: x = e1 mod q, src = e1 (i64)
 //            2: x = u mapped 0 -> q-1, 1 -> 0, 2 -> 1, src = u (u8)
-//   MULM     MUL with aux in Montgomery form (launch_to_montgomery); x in [0, 2q)
-//   DOTM     DOT with the key in Montgomery form; x in [0, 3q)
+//   MULM     MUL with aux prepared (launch_to_montgomery: Montgomery form, unchanged
+//            on pm limbs); x in [0, 2q), on pm limbs [0, 4q)
+//   DOTM     DOT with the key prepared; x in [0, 3q), on pm limbs [0, 5q)
 enum NttLoad : uint32_t {
   NTT_LOAD_NONE = 0,
   NTT_LOAD_MUL = 1,
@@ -39,8 +40,8 @@ enum NttLoad : uint32_t {
 //   NONE         dst[i] = y
 //   RESCALE      dst[i] = (aux[i] - y) * q_last^{-1} mod q
 //   MUL_RESCALE  dst[i] = (aux[i] * aux2[i] - y) * q_last^{-1} mod q
-//   MONT         dst[i] = y 2^64 mod q (Montgomery form), and aux[i] = y when the
-//                job's aux is not null (aux is then written, not read)
+//   MONT         dst[i] = y prepared (y 2^64 mod q, Montgomery form; y on pm limbs),
+//                and aux[i] = y when the job's aux is not null (then written, not read)
 // With y = NTT_q(c_last mod q) the rescale forms are the rescale of
 // ciphertext.rs:476-535 in the evaluation domain: the NTT is linear mod q, so
 //   NTT_q((c_q - (c_last mod q)) * inv) = (C_q - NTT_q(c_last mod q)) * inv
