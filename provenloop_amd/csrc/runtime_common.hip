@@ -2,6 +2,7 @@
 // lifetime, sampler band flags, NTT dispatch, context tables, and the
 // encode, encrypt, product, rescale and decrypt pipelines the entry points
 // queue on a context's stream.
+#include "launch_rules.h"
 #include "runtime.h"
 
 namespace thrt {
@@ -779,14 +780,11 @@ void check_decrypt_args(th_ctx* c, const th_ct* const* cts, size_t count, const 
   for (size_t i = 0; i < count; ++i) check_ct(c, cts[i]);
 }
 
-// D2H through the staging ring, then wait: polling (wait_stream) up to 256 KiB,
-// where the wait's latency counts (a layer of per-call decryptions, 64 KiB each:
-// 890 -> 830 us a pass); the poll's queries slow a larger copy down (key export,
-// 512 KiB and 1 MiB: 205 -> 219 us), which waits in the runtime.
+// D2H through the staging ring, then wait (poll_download: how).
 void download(th_ctx* c, void* dst, const void* src_dev, size_t bytes) {
   void* h = c->ring.reserve(bytes, c->stream);
   HIPCHK(hipMemcpyAsync(h, src_dev, bytes, hipMemcpyDeviceToHost, c->stream));
-  if (bytes <= (256u << 10))
+  if (poll_download(bytes))
     wait_stream(c);
   else
     HIPCHK(hipStreamSynchronize(c->stream));
