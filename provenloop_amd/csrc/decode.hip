@@ -17,6 +17,7 @@
 // stages combine the parts element-wise in a second kernel, which also forms
 // the ZeRo-MOAI segment sums.
 #include "fft_device.h"
+#include "launch_rules.h"
 #include "poly_kernels.h"
 
 namespace th {
@@ -64,10 +65,6 @@ __device__ __forceinline__ double coeff_centred(const DecodeJob& jb, const Decod
 }
 
 constexpr int DEC_THREADS = 1024;
-// Parts are added while a batch makes fewer workgroups than CUs: 112 decodes
-// at N = 16384 (the batched operations of 28 inputs) took 638 us a pass with
-// 256, 676 with 128 and 691 with the encoder's 512.
-constexpr uint32_t DEC_FILL = 256;
 
 // The in-part stages of part blockIdx.x of job blockIdx.y, over the elements
 // whose bit-reversed position lies in the part: the coefficient's f64 value
@@ -284,7 +281,7 @@ hipError_t launch_decode(const DecodeJob* jobs, uint32_t njobs, const DecodeCons
                          uint32_t d, uint32_t cols, hipStream_t s) {
   if (!njobs) return hipSuccess;
   if (cols == 0) {  // slots only
-    const uint32_t lp = fft_batch_parts_log(logn, njobs, DEC_FILL), M = (1u << logn) >> lp;
+    const uint32_t lp = decode_parts_log(logn, njobs), M = (1u << logn) >> lp;
     const uint32_t threads = M / 8 < 64 ? 64 : (M / 8 > DEC_THREADS ? DEC_THREADS : M / 8);
     const uint32_t fin = lp >= 2 ? M << (lp - 2) : M;
     const size_t lds = fft_part_lds(logn, lp);

@@ -12,6 +12,7 @@
 // All f64 steps round exactly as on the host (-ffp-contract=off, host
 // twiddles), so m is bit-identical to the reference encoder's.
 #include "fft_device.h"
+#include "launch_rules.h"
 #include "sample_device.h"
 
 namespace th {
@@ -276,10 +277,7 @@ hipError_t launch_encode(const EncodeJob* jobs, uint32_t njobs, const BarrettCon
   if (sample && seeds)
     for (uint32_t i = 0; i < njobs; ++i) sb.v[i] = seeds[i];
   const int use_sb = seeds != nullptr;
-  // 672 encodes of N=16384 per CryptoMOE token: the token measured 0.656 ms
-  // with parts of 4096 values against 0.697 ms with 8192, 0.675 ms with 2048
-  // and 0.727 ms with 1024
-  const uint32_t lp = fft_batch_parts_log(logn, njobs, 512);
+  const uint32_t lp = encode_parts_log(logn, njobs);
   const uint32_t M = n >> lp;
   const size_t lds = fft_part_lds(logn, lp);
   // dit_stages_reg needs 8 values per thread at most

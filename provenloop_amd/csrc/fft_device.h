@@ -209,16 +209,6 @@ __device__ __forceinline__ void combine_parts(GPtr<double> Pd, uint32_t k, uint3
   }
 }
 
-// log2 of the parts a batch of njobs transforms is cut into: parts of at most
-// 4096 values (two workgroups' LDS per CU), and more of them (up to 16, of at
-// least 1024 values) while the batch makes fewer than `fill` workgroups. The
-// parts are independent workgroups and the result is the same for any split.
-inline uint32_t fft_batch_parts_log(uint32_t logn, uint32_t njobs, uint32_t fill) {
-  const uint32_t lp_min = fft_parts_log(logn);
-  uint32_t lp = logn > 12 && logn - 12 > lp_min ? logn - 12 : lp_min;
-  while (lp < 4 && logn - lp > 10 && njobs * (1u << lp) < fill) ++lp;
-  return lp;
-}
 // LDS of one part's workgroup: padded values, and twiddles with 8 or more parts.
 inline size_t fft_part_lds(uint32_t logn, uint32_t lp) {
   const uint32_t M = (1u << logn) >> lp;

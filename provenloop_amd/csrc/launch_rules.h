@@ -17,4 +17,38 @@ namespace th {
 // makes no difference.
 constexpr bool poll_download(size_t bytes) { return bytes > (16u << 10) && bytes <= (256u << 10); }
 
+// A transform of N complex values (encoder, decoder) is cut into 2^lp parts of
+// N / 2^lp values, one workgroup each, of an eighth as many threads (64 to
+// 1024); the result is the same for any split. From 8 parts on a part stages
+// its twiddles in LDS beside its values (fft_part_lds): 4096 values take 72
+// KiB, 136 with the twiddles, so at N = 32768 a CU holds one workgroup of 512
+// threads; 8192 values take 144 KiB with 1024 threads.
+//
+// Encodes: parts of at most 4096 values, and more of them (up to 16, of at
+// least 1024 values) while the batch makes fewer than 512 workgroups. 672
+// encodes of N = 16384 per CryptoMOE token: the token measured 0.656 ms with
+// parts of 4096 values against 0.697 ms with 8192, 0.675 ms with 2048 and
+// 0.727 ms with 1024.
+constexpr uint32_t encode_parts_log(uint32_t logn, uint32_t njobs) {
+  uint32_t lp = logn <= 12 ? 0 : logn - 12;
+  while (lp < 4 && logn - lp > 10 && njobs * (1u << lp) < 512) ++lp;
+  return lp;
+}
+
+// Decodes: parts of 4096 values, 8192 at N = 32768, and more of them (up to 16,
+// of at least 1024 values) while they are still one workgroup per CU. Batches
+// with 4 / 8 / 16 parts each:
+//   N = 32768, 64 decodes     92 / 107 / 112 us (CRT 119 / 143 / 145)
+//   N = 32768, 256            267 / 307 / 314   (CRT 365 / 444 / 424)
+//   N = 32768, 24             69 / 63 / 69      (CRT 85 / 81 / 87)
+//   N = 32768, 16             66 / 59 / 59
+//   N = 16384, 33             57 / 61 / 65      (CRT 70 / 77 / 83)
+//   N = 16384, 16             52 / 49 / 49
+constexpr uint32_t DECODE_FILL = 256;  // workgroups: the CU count
+constexpr uint32_t decode_parts_log(uint32_t logn, uint32_t njobs) {
+  uint32_t lp = logn <= 12 ? 0 : logn == 13 ? 1 : 2;
+  while (lp < 4 && logn - lp > 10 && ((uint64_t)njobs << (lp + 1)) <= DECODE_FILL) ++lp;
+  return lp;
+}
+
 }  // namespace th

@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,count", [(1024, 1), (1024, 3), (2048, 1), (4096, 2), (8192, 1), (8192, 33), (8192, 70),
-                                     (16384, 1), (16384, 33), (16384, 65), (16384, 130), (32768, 1), (32768, 33)])
+                                     (16384, 1), (16384, 33), (16384, 65), (16384, 130), (32768, 1), (32768, 17),
+                                     (32768, 33)])
 def test_batch_decrypt_matches_oracle(n, count):
     q = orc.default_chain(max(n, 8192))
     eng, ref = tensafe_he.CkksContext(n, moduli=q), orc.Context(n, moduli=q)

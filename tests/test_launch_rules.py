@@ -27,3 +27,22 @@ def test_small_downloads_wait_in_the_runtime(evaluate):
     sizes = [0, 4, 8, 256, 16 << 10, (16 << 10) + 1, 32 << 10, 64 << 10, 128 << 10, 256 << 10, (256 << 10) + 1]
     got = evaluate([f"th::poll_download({b})" for b in sizes])
     assert got == [0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 0]
+
+
+def test_decodes_are_cut_into_at_most_one_part_per_cu(evaluate):
+    """Parts of 4096 values (8192 at N = 32768, whose parts of 4096 leave a CU one small workgroup), more only while
+    the batch has no more parts than the GPU has CUs; every part fits a workgroup of 8 values a thread."""
+    cases = [(logn, jobs) for logn in range(10, 16) for jobs in (1, 8, 15, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257, 5000)]
+    got = dict(zip(cases, evaluate([f"th::decode_parts_log({n}, {j})" for n, j in cases])))
+    base = {10: 0, 11: 0, 12: 0, 13: 1, 14: 2, 15: 2}
+    for (logn, jobs), lp in got.items():
+        assert base[logn] <= lp <= 4 and 1 << logn >> lp <= 8192
+        assert lp == base[logn] or (jobs << lp <= 256 and logn - lp >= 10)
+        if lp < 4 and logn - lp > 10:
+            assert jobs << (lp + 1) > 256
+    assert [got[15, j] for j in (16, 17, 32, 33, 64, 256)] == [4, 3, 3, 2, 2, 2]
+
+
+def test_encodes_fill_two_workgroups_per_cu(evaluate):
+    cases = [(13, 1), (13, 64), (13, 255), (13, 256), (14, 28), (14, 64), (14, 128), (14, 672), (15, 28), (15, 64), (10, 1)]
+    assert evaluate([f"th::encode_parts_log({n}, {j})" for n, j in cases]) == [3, 3, 2, 1, 4, 3, 2, 2, 4, 3, 0]
