@@ -534,12 +534,32 @@ __device__ __forceinline__ uint32_t column_part(uint32_t p) {
   }
 }
 
+// Wavefronts per SIMD of a split kernel, or `any`. The plain inverse passes on
+// pm limbs need 92 to 94 registers, which allows five, but their LDS holds 18
+// workgroups on a CU, so SIMDs hold four or five, in rounds that do not end
+// together: 16 on a CU through the LDS size change nothing, four on each SIMD
+// do, and in the column pass, whose wavefronts each store 16 lines of the
+// natural layout, three. A pass of 64 transforms of 4 limbs at N = 32768 with
+// the copy before it: 75.4 us with neither, 73.0 with four in both, 71.4 with
+// three in the column pass, 73.5 with three in the row pass; 256 of them 334,
+// 326, 319, 335; N = 16384, 256: 174, 168, 161, 169. In place on data the
+// caches hold the passes stay within 2 %. IntArith's take 99 registers and more,
+// four wavefronts, by themselves.
+constexpr int MAX_WAVES = 8;
+template <class BIG, bool INV, bool COLUMN, uint32_t LD, uint32_t ST>
+constexpr int split_waves(int any) {
+  if (!std::is_same_v<BIG, PmArith> || !INV || LD != NTT_LOAD_NONE || ST != NTT_STORE_NONE) return any;
+  return COLUMN ? 3 : 4;
+}
+
 // Workgroup b works on part b % PARTS of job b / PARTS. The pass that reads
 // the transform's input applies the fused load operation and the forward
 // row pass the fused store operation; otherwise passes read and write the
 // destination only.
 template <class BIG, int LOGN, bool INV, bool COLUMN, uint32_t LD, uint32_t ST, bool STREAM = false>
-__global__ __launch_bounds__(64) void ntt_split_kernel(NttArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
+    split_waves<BIG, INV, COLUMN, LD, ST>(1), split_waves<BIG, INV, COLUMN, LD, ST>(MAX_WAVES)))) void
+ntt_split_kernel(NttArgs a) {
   using S = Split<LOGN>;
   // the forward row pass with a fused rescale store, and the inverse row pass
   // with the product in its loads, also hold one register pass's twiddles
