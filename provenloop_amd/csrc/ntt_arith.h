@@ -154,12 +154,19 @@ struct Fp64Arith {
 
 // f.template operator()<A>() with the arithmetic of limb lc (uniform over the
 // workgroup): Fp64Arith below 2^41, else the chain's BIG (PmArith or IntArith).
-template <class BIG, class F>
+// APART: nothing that both begin or end with is merged (the compiler hoists and
+// sinks it, and holds its registers through either).
+template <class BIG, bool APART = false, class F>
 __device__ __forceinline__ void with_arith(const LimbConst& lc, F&& f) {
-  if (lc.kind == LIMB_FP64)
+  if (lc.kind == LIMB_FP64) {
+    if constexpr (APART) asm volatile("; fp64 limb");
     f.template operator()<Fp64Arith>();
-  else
+    if constexpr (APART) asm volatile("; fp64 limb, end");
+  } else {
+    if constexpr (APART) asm volatile("; limb above 2^41");
     f.template operator()<BIG>();
+    if constexpr (APART) asm volatile("; limb above 2^41, end");
+  }
 }
 
 // a times a prepared operand b (launch_to_montgomery) mod q: below 2q, or on

@@ -82,16 +82,12 @@ __device__ __forceinline__ void store_hint(T v, GMut<T> p) {
   else
     *p = v;
 }
-// The 16 intermediate values at buf[at(k)].
-template <bool STREAM, class A, class At>
-__device__ __forceinline__ void load_raw(typename A::V (&x)[16], const A& ar, GPtr<uint64_t> buf, const At& at) {
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    if constexpr (STREAM)
-      x[k] = ar.unraw(__builtin_nontemporal_load(&buf[at(k)]));
-    else
-      x[k] = ar.unraw(buf[at(k)]);
-  }
+template <bool STREAM, class T>
+__device__ __forceinline__ T load_hint(GPtr<T> p) {
+  if constexpr (STREAM)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
 }
 
 __device__ __forceinline__ uint32_t pad16(uint32_t e) { return e + (e >> 4); }
@@ -388,7 +384,8 @@ __device__ __forceinline__ void row_fwd_regs(typename A::V (&x)[16], const uint6
   const GPtr<uint64_t> gbuf = gld(buf);
   const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd));
   const GPtr<typename A::Tw> tr = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd_row));
-  load_raw<STREAM>(x, ar, gbuf + jbase, p1);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) x[k] = ar.unraw(load_hint<STREAM>(&gbuf[jbase + p1(k)]));
   fwd_stages<LOGN, CB - 4, CB - 1, CB - 4>(x, jbase + p1(0), tw, ar);
   wave_exchange(x, lds, p1, p2);
   // the stages on the P2 register bits read the row table (one load of
@@ -423,7 +420,8 @@ __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint6
   };
   if constexpr (!INV) {
     const GPtr<typename A::Tw> tw = gld(reinterpret_cast<const typename A::Tw*>(lc.fwd));
-    load_raw<STREAM>(x, ar, (GPtr<uint64_t>)gdst + jbase, p1);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = ar.unraw(load_hint<STREAM>((GPtr<uint64_t>)&gdst[jbase + p1(k)]));
     if constexpr (SOp::NAUX > 0) {
       // The store's operands and outputs in pairs of adjacent positions per
       // lane: register k is position h(k) = 2 lane + (k & 1) + 128 (k >> 1)
@@ -611,8 +609,16 @@ ntt_split_kernel(NttArgs a) {
 // forward passes (workgroup b: part b % PARTS of forward job b / PARTS), so
 // the launch takes one inverse and one forward pass instead of the inverse
 // and nf forward passes in turn.
+// Wavefronts per SIMD: three. With Shoup products that needs the arithmetics'
+// code kept apart (with_arith) at N <= 16384 (160 to 164 registers, against 183
+// to 190 and two wavefronts, or 16 registers spilled at three: 200 products
+// 282 us against 291 and 296), and spills all the same at N = 32768, which has
+// two (64 products on 8 limbs: 276 us, 293 at three).
+template <class BIG, int LOGN>
+constexpr bool RESCALE_APART = std::is_same_v<BIG, IntArith> && LOGN < 15;
 template <class BIG, int LOGN, bool STREAM>
-__global__ __launch_bounds__(64, 3) void rescale_column_kernel(NttArgs inv, NttArgs fwd, uint32_t nf, uint32_t fan) {
+__global__ __launch_bounds__(64, (std::is_same_v<BIG, PmArith> || LOGN < 15 ? 3 : 1))
+void rescale_column_kernel(NttArgs inv, NttArgs fwd, uint32_t nf, uint32_t fan) {
   using S = Split<LOGN>;
   __shared__ uint64_t lds[S::LDS];
   const uint32_t unit = blockIdx.x / S::PARTS;  // inverse job, or forward job with fan
@@ -622,7 +628,7 @@ __global__ __launch_bounds__(64, 3) void rescale_column_kernel(NttArgs inv, NttA
   const NttJob ij = inv.jobs[job];
   const LimbConst& lci = inv.lc[ij.limb];
   uint64_t c[16];  // canonical last-limb coefficients of this wavefront's columns (Q1)
-  with_arith<BIG>(lci, [&]<class A>() {
+  with_arith<BIG, RESCALE_APART<BIG, LOGN>>(lci, [&]<class A>() {
     const A ar(lci);
     typename A::V x[16];
     column_inv_regs<LOGN>(x, ij.dst, lci, m, ar, lds);
@@ -639,7 +645,7 @@ __global__ __launch_bounds__(64, 3) void rescale_column_kernel(NttArgs inv, NttA
     // hoisting per-coefficient terms out of the loop into extra registers
 #pragma unroll
     for (int k = 0; k < 16; ++k) c[k] = opaque_u64(c[k]);
-    with_arith<BIG>(lcf, [&]<class A>() {
+    with_arith<BIG, RESCALE_APART<BIG, LOGN>>(lcf, [&]<class A>() {
       const A ar(lcf);
       typename A::V x[16];
 #pragma unroll

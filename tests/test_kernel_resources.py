@@ -79,3 +79,24 @@ def test_plain_inverse_passes_keep_their_wavefronts(kernels, logn):
     for column, waves in ((0, 4), (1, 3)):
         name = f"16ntt_split_kernelI{PM}Li{logn}ELb1ELb{column}ELj0ELj0ELb0E"
         assert [w for w, _ in _find(kernels, name).values()] == [waves]
+
+
+def test_split_kernels_do_not_spill(kernels):
+    """None of them, on either arithmetic above 2^41."""
+    for name, (_, scratch) in _find(kernels, "ntt_split_kernel|rescale_column_kernel|encrypt_row_kernel|2rd_").items():
+        assert scratch == 0, name
+
+
+@pytest.mark.parametrize("kind,logn,waves", [(PM, 13, 3), (PM, 14, 3), (PM, 15, 3), (INT, 13, 3), (INT, 14, 3), (INT, 15, 2)])
+def test_rescale_columns_keep_their_wavefronts(kernels, kind, logn, waves):
+    for w, _ in _find(kernels, f"21rescale_column_kernelI{kind}Li{logn}E").values():
+        assert w == waves
+
+
+@pytest.mark.parametrize("kind", [PM, INT])
+@pytest.mark.parametrize("logn", [13, 14, 15])
+def test_forward_rows_and_encryption_keep_their_wavefronts(kernels, kind, logn):
+    """Four per SIMD: the plain forward row pass and the encryption's."""
+    for name in (f"16ntt_split_kernelI{kind}Li{logn}ELb0ELb0ELj0ELj0ELb0E", f"18encrypt_row_kernelI{kind}Li{logn}E"):
+        for w, _ in _find(kernels, name).values():
+            assert w >= 4
