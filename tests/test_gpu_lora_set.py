@@ -456,10 +456,15 @@ def test_lora_set_split_rescale_decrypt_equals_whole(env):
     (8192, None),
     (32768, None),
     (16384, [1099507695617, 1099506515969, 1152921504598720513]),
+    (16384, [1125899904679937, 1099507695617, 1152921504598720513]),
+    (8192, [1152921504539017217, 1099507695617, 1152921504538951681]),
+    (32768, [1152921504539017217, 1099507695617, 1152921504538951681]),
 ])
 def test_lora_set_split_rescale_decrypt_matches_oracle(n, moduli):
-    """The split-kernel rescale-decrypt at log N = 13 and 15 (default chains) and on a 40-bit
-    limb 0 (FP64 transforms, last-limb values reduced by Barrett) against the oracle."""
+    """The split-kernel rescale-decrypt at log N = 13 and 15 (default chains), on a 40-bit limb 0
+    (FP64 transforms, last-limb values reduced by Barrett), and with Shoup products on limb 0
+    and the last limb (a 50-bit prime, and primes just below 2^60 - 2^26, the end of the
+    folded products' range), against the oracle."""
     eng = tensafe_he.CkksContext(n, moduli=moduli)
     ref = orc.Context(n, moduli=moduli) if moduli else orc.Context(n)
     sk, rsk = eng.keygen(seed=7), ref.keygen(7)

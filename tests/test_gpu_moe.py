@@ -179,6 +179,27 @@ def test_moe_set_gates_matches_oracle_per_token(env):
             assert np.linalg.norm(g - e) <= 1e-3 * np.linalg.norm(e)
 
 
+def test_moe_set_gates_with_shoup_products():
+    """Regating (the plaintexts' prepared copy of an integer limb in Montgomery form) and the tokens after it on a
+    chain whose large primes lie just below 2^60 - 2^26, outside the folded products' range, against the oracle."""
+    q = [1152921504539017217, 1099507695617, 1152921504538951681]
+    eng, ref = tensafe_he.CkksContext(8192, moduli=q), orc.Context(8192, moduli=q)
+    sk, rsk = eng.keygen(seed=53), ref.keygen(53)
+    pk, rpk = eng.keygen_public(sk, seed=54), ref.keygen_public(rsk, 54)
+    rng = np.random.default_rng(29)
+    proj, g0 = _experts(rng, 1, d=512, rank=9, d_outs=(24, 8))
+    ls = zero_moai.LoraSet(eng, 1, proj, gates=g0)
+    for t in range(2):
+        H = rng.normal(size=(1, 512)) * 0.1
+        gt = np.array([zero_moai.softmax_gate(100 * t + j, K) for j in range(len(proj))])
+        ls.set_gates(gt)
+        got, got_sums = ls.deltas(pk, sk, H, [210 + t], with_intermediates=True)
+        exp, exp_sums = _oracle(ref, rpk, rsk, H, [210 + t], proj, gt)
+        assert np.max(np.abs(got_sums - exp_sums)) <= 1e-9 * max(1.0, np.max(np.abs(exp_sums)))
+        for g, e in zip(got, exp):
+            assert np.linalg.norm(g - e) <= 1e-3 * np.linalg.norm(e)
+
+
 def test_moe_set_gates_errors(env):
     eng = env[0]
     rng = np.random.default_rng(27)
