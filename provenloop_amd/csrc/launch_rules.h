@@ -1,5 +1,5 @@
-// Rules on sizes that need no device, kept apart from HIP so that a host
-// program can evaluate them (tests/test_launch_rules.py).
+// Rules on sizes, and the job lists' ring, that need no device: kept apart from
+// HIP so that a host program can evaluate them (tests/test_launch_rules.py).
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
@@ -50,5 +50,29 @@ constexpr uint32_t decode_parts_log(uint32_t logn, uint32_t njobs) {
   while (lp < 4 && logn - lp > 10 && ((uint64_t)njobs << (lp + 1)) <= DECODE_FILL) ++lp;
   return lp;
 }
+
+// Places for short job lists in a ring of `cap` bytes, handed out in turn on
+// 256-byte boundaries. A list that does not fit behind the last one starts a
+// new lap, for which drain() first waits for everything queued so far: a place
+// is never handed out again while a queued kernel may read it.
+class SlotRing {
+ public:
+  explicit constexpr SlotRing(size_t cap) : cap_(cap) {}
+  // the offset of a place of `bytes` <= cap bytes
+  template <class Drain>
+  size_t place(size_t bytes, Drain&& drain) {
+    const size_t step = (bytes + 255) & ~(size_t)255;
+    if (off_ + step > cap_) {
+      drain();
+      off_ = 0;
+    }
+    const size_t at = off_;
+    off_ += step;
+    return at;
+  }
+
+ private:
+  size_t cap_, off_ = 0;
+};
 
 }  // namespace th

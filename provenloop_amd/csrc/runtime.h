@@ -38,6 +38,7 @@
 
 #include "encode_sample.h"
 #include "host_math.h"
+#include "launch_rules.h"
 #include "poly_kernels.h"
 #include "tensafe_he.h"
 
@@ -151,9 +152,8 @@ class StagingRing {
 // Short job lists (a few descriptors) in pinned pages that the kernels read
 // themselves, instead of a host-to-device copy that is a launch of its own:
 // about 3 us on the GPU and the gaps around it, against about 1 us more on the
-// reading kernel's first access. Slots are handed out in turn; a lap of the
-// 1 MiB (4096 slots) drains the stream first, so a slot is never rewritten
-// while a queued kernel may read it, and no call holds more than a few.
+// reading kernel's first access. A lap of the 1 MiB (4096 lists of up to 256
+// bytes) drains the stream, and no call holds more than a few (SlotRing).
 class JobSlots {
  public:
   static constexpr size_t SLOT = 512, CAP = 1u << 20;  // largest list, ring size
@@ -167,21 +167,15 @@ class JobSlots {
   }
   // the device address of a copy of bytes <= SLOT at src
   void* put(const void* src, size_t bytes, hipStream_t s) {
-    const size_t step = (bytes + 255) & ~(size_t)255;
-    if (off_ + step > CAP) {
-      HIPCHK(hipStreamSynchronize(s));
-      off_ = 0;
-    }
-    memcpy((char*)host_ + off_, src, bytes);
-    void* d = (char*)dev_ + off_;
-    off_ += step;
-    return d;
+    const size_t at = ring_.place(bytes, [&] { HIPCHK(hipStreamSynchronize(s)); });
+    memcpy((char*)host_ + at, src, bytes);
+    return (char*)dev_ + at;
   }
 
  private:
   void* host_ = nullptr;
   void* dev_ = nullptr;
-  size_t off_ = 0;
+  th::SlotRing ring_{CAP};
 };
 
 // Parallel loop over independent host work items (sampling, encoding).

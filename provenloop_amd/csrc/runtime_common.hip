@@ -2,7 +2,6 @@
 // lifetime, sampler band flags, NTT dispatch, context tables, and the
 // encode, encrypt, product, rescale and decrypt pipelines the entry points
 // queue on a context's stream.
-#include "launch_rules.h"
 #include "runtime.h"
 
 namespace thrt {

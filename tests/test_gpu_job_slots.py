@@ -1,9 +1,11 @@
 """Short job lists stay in a ring of pinned slots that the kernels read.
 
-More operations than the ring has slots (4096 lists of up to 256 bytes), queued
-without waiting, so slots are handed out again after a lap: the running sum of
-a ciphertext with itself must still be exact, and lists on both sides of the
-slot size (a batch of one product, and one of many) give the same residues.
+More operations than the ring has slots (4096 lists of up to 256 bytes), so
+slots are handed out again after a lap: the running sum of a ciphertext with
+itself must still be exact, and lists on both sides of the slot size (a batch
+of one product, and one of many) give the same residues. That a lap waits for
+what is queued before a slot is rewritten is tested on the host
+(test_launch_rules.py): calls come too slowly to overtake the GPU by a lap.
 """
 import numpy as np
 import pytest

@@ -1,4 +1,4 @@
-"""The dispatch rules that need no device (launch_rules.h), evaluated by a host program at the lines they draw."""
+"""The dispatch rules and the job lists' ring (launch_rules.h), which need no device, evaluated by host programs."""
 import os
 import subprocess
 
@@ -8,18 +8,24 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 
 @pytest.fixture(scope="module")
-def evaluate(tmp_path_factory):
-    """evaluate(["expression", ...]) -> their values, as integers."""
+def program(tmp_path_factory):
+    """program(body of main) -> the integers it prints."""
 
-    def run(exprs):
+    def run(body):
         d = tmp_path_factory.mktemp("rules")
         src, exe = d / "rules.cpp", d / "rules"
-        src.write_text('#include "launch_rules.h"\n#include <stdio.h>\nint main() {\n'
-                       + "".join(f'  printf("%lld\\n", (long long)({e}));\n' for e in exprs) + "}\n")
+        src.write_text('#include "launch_rules.h"\n#include <stdio.h>\n#include <utility>\n#include <vector>\n'
+                       "int main() {\n" + body + "}\n")
         subprocess.run(["g++", "-std=c++20", "-Wall", "-Werror", "-I", CSRC, str(src), "-o", str(exe)], check=True)
         return [int(v) for v in subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()]
 
     return run
+
+
+@pytest.fixture(scope="module")
+def evaluate(program):
+    """evaluate(["expression", ...]) -> their values, as integers."""
+    return lambda exprs: program("".join(f'  printf("%lld\\n", (long long)({e}));\n' for e in exprs))
 
 
 def test_small_downloads_wait_in_the_runtime(evaluate):
@@ -46,3 +52,27 @@ def test_decodes_are_cut_into_at_most_one_part_per_cu(evaluate):
 def test_encodes_fill_two_workgroups_per_cu(evaluate):
     cases = [(13, 1), (13, 64), (13, 255), (13, 256), (14, 28), (14, 64), (14, 128), (14, 672), (15, 28), (15, 64), (10, 1)]
     assert evaluate([f"th::encode_parts_log({n}, {j})" for n, j in cases]) == [3, 3, 2, 1, 4, 3, 2, 2, 4, 3, 0]
+
+
+def test_job_lists_are_not_rewritten_before_a_drain(program):
+    """Every place handed out is clear of all the places handed out since the last drain, at the library's capacity
+    and at small ones, with lists of mixed sizes; and laps do come round."""
+    overlaps, laps = program("""
+  long long overlaps = 0, laps = 0;
+  unsigned x = 1;
+  for (size_t cap : {size_t(512), size_t(768), size_t(4096), size_t(1) << 20}) {
+    th::SlotRing ring(cap);
+    std::vector<std::pair<size_t, size_t>> queued;  // what kernels may still read
+    for (int i = 0; i < 20000; ++i) {
+      x = x * 1664525u + 1013904223u;
+      const size_t bytes = 1 + (x >> 8) % 512;
+      const size_t at = ring.place(bytes, [&] { queued.clear(); ++laps; });
+      if (at + bytes > cap || at % 256) ++overlaps;
+      if (i < 9000 || cap < 5000)
+        for (auto& q : queued) overlaps += at < q.first + q.second && q.first < at + bytes;
+      queued.push_back({at, bytes});
+    }
+  }
+  printf("%lld %lld\\n", overlaps, laps);
+""")
+    assert overlaps == 0 and laps > 1000
