@@ -401,7 +401,8 @@ struct StoreOp {
   template <class A>
   __device__ __forceinline__ uint64_t apply_prep(const A& ar, typename A::V x, uint64_t cp) const {
     if constexpr (std::is_same_v<A, Fp64Arith> && NAUX > 0) {
-      // (c - x) * inv with the output as it is: |x| < 16 q, |c - x| < 2^46
+      // (c - x) * inv with the output as it is: |x| < 9 q + 2^32 (the input,
+      // reduce_u64_f64, and at most 15 stages of 0.51 q), so |c - x| < 2^46
       const double c = __builtin_bit_cast(double, cp);
       const double r = mulmod_f64(c - x, rc.inv_d, rc.inv_dq, rc.qd);
       return f64_to_u64(r < 0.0 ? r + rc.qd : r);

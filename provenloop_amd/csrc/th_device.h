@@ -309,7 +309,8 @@ __device__ __forceinline__ double mulmod_f64(double x, double w, double wq, doub
 }
 
 // A residue of any c < 2^61 modulo a limb q_l below 2^41, as an exact double
-// below 0.52 q_l + 2^32 in magnitude, the forward transforms' input: with c =
+// of magnitude below 0.76 q_l + 2^32 (0.52 q_l + 2^32 from q_l = 2^21 on, 2^32
+// being most of it for a small q_l), the forward transforms' input: with c =
 // ch 2^32 + cl (ch < 2^29) and quot = rint(ch 2^32 / q_l), ch - quot q_l / 2^32
 // is an exact multiple of 2^-32 (one FMA), and times 2^32 plus cl the residue
 // (another). Six instructions; through 2^32 mod q_l and corrected into [0,
