@@ -33,12 +33,12 @@ void launch_jobs_ntt(th_ctx* c, bool inverse, const NttJob* jobs, uint32_t n, Nt
 
 // Queue the plaintexts and mixed B of a mixture set for its gates (set->d_gates,
 // n_proj x k): every batch's plaintext is sum_x encode_to_ntt(g_x * A_x rows)
-// (the encoder and transforms of th_encode_to_ntt), in Montgomery form (and
-// plain where a token reads it), and B = sum_x g_x B_x. The encoder gates the
+// (the encoder and transforms of th_encode_to_ntt), prepared (and plain
+// where a token reads it), and B = sum_x g_x B_x. The encoder gates the
 // experts' packed rows as it reads them, and its last launch sums the k
 // experts' residues of each batch (the k encoded residue polynomials summed
 // mod q_l); each batch's forward transform then runs once per limb, in place,
-// and writes the Montgomery form in its store (NTT_STORE_MONT). The
+// and writes the prepared form in its store (NTT_STORE_MONT). The
 // transform is linear mod q_l, so this is the sum of the k transforms,
 // residue by residue. Only the limbs a token reads are formed.
 void queue_regate(OpScope& sc, th_lora* set) {
@@ -214,8 +214,8 @@ void build_lora(th_lora* set, const uint32_t* input_of, const uint32_t* ranks, c
     set->d_gates = (double*)set->alloc((size_t)set->n_proj * k * 8);
     // A complete token (ct x pt on every limb) reads every limb of the
     // plaintexts in plain form (the rescale's store, the products) and limb
-    // L-1 in Montgomery form (the rescale's inverse loads); a fused token
-    // reads limbs 0..nl-1 and L-1 in Montgomery form: the regated plaintexts
+    // L-1 prepared (the rescale's inverse loads); a fused token
+    // reads limbs 0..nl-1 and L-1 prepared: the regated plaintexts
     // are formed on every limb, in both forms.
     set->moe_limbs = L >= 32 ? ~0u : (1u << L) - 1;
     std::vector<NttJob> mj;

@@ -15,8 +15,9 @@
 // NTT_WHOLE_MAX_JOBS = 256 (the CU count) use the first, the others the second
 // (the segment-sum epilogue exists in the first only).
 // (Those figures are of Shoup products on the 60-bit limbs. With the folded
-// products the 256-transform batch of 64 polynomials measured 35.7 us a pass
-// with its copy on the whole kernel and 40.0 on the split ones: the same side.)
+// products the 256-transform batch of 64 polynomials measured 35.7 us with the
+// copy before it on the whole kernel and 40.0 on the split ones, one stream by
+// itself: the same side.)
 #include "ntt_kernels.h"
 
 namespace th {

@@ -42,8 +42,15 @@
 // (N = 32768, 3.3 GB of it): encrypt column pass 140 -> 106 us,
 // rescale column kernel 1159 -> 1108, fused-rescale row pass 1868 -> 1766.
 // Launches that fit keep plain accesses: with the hint on all of them a
-// CryptoMOE token went from 692 to 713 us, and the batched inverse at N = 32768
-// (hint on its passes) from 82 to 88-98.
+// CryptoMOE token (176 MB) went from 692 to 713 us, and the batched inverse at
+// N = 32768, 64 transforms of 4 limbs (hint on its passes), lost 7 to 20 %.
+// Tokens above the line, without the hint / with it: N = 32768, 8 limbs, 80
+// products (294 MB) 453 / 417 us, 128 (470 MB) 665 / 608, 256 (940 MB) 1205 /
+// 1083; 4 limbs, 176 (277 MB) 536 / 503, 256 (403 MB) 720 / 675, 448 (705 MB)
+// 1166 / 1114; N = 16384, 352 (277 MB) 569 / 544, 576 (453 MB) 874 / 837;
+// encryptions at N = 32768, 8 limbs, 44 (277 MB) 615 / 553, 96 (604 MB) 1259 /
+// 1063. Below it, down to 176 MB, the hint wins on such tokens as well (64
+// products on 8 limbs, 235 MB, 390 / 359) and loses on the CryptoMOE one.
 // Column-pass wavefronts 2m and 2m+1 share the 128-byte lines of the
 // natural layout; they are given workgroup ids that the dispatcher sends to
 // the same XCD (ids are dealt round-robin over the 8 XCDs), so the second
@@ -429,9 +436,12 @@ __device__ __forceinline__ void row_pass(const uint64_t* __restrict__ src, uint6
       // instructions of the lane-contiguous layout (this pass is bound by
       // the CUs' vector-memory address processing more than by its
       // arithmetic). The operands are requested after the first register
-      // pass and combined after the exchange that follows it: held from the
-      // start, they cost the kernel a wavefront per SIMD (156 VGPRs against
-      // 127), which measured slower (106.3 against 104.1 us per token).
+      // pass and combined after the exchange that follows it. (With Shoup
+      // products, requesting them at the start took 156 VGPRs against 127, a
+      // wavefront per SIMD less, and 106.3 us per token against 104.1. With
+      // folded products the kernel has 216-219 VGPRs and two wavefronts per
+      // SIMD: its product in the store and the limbs' FP64 code, 130, are in
+      // one kernel. Capped at 128 it spills: 111 -> 154 us.)
       auto h = [&](uint32_t k) { return (l << 1) + (k & 1) + ((k >> 1) << 7); };
       using U2 = uint64_t __attribute__((ext_vector_type(2)));
       typename SOp::Aux v[16];
@@ -803,7 +813,7 @@ __global__ __launch_bounds__(192) void encrypt_row_kernel(NttArgs a, const uint6
       }
     }
     if (form_d) {
-      // D = c0 + c1 s in [0, 3q) (the key prepared for fixed_mul), at input i's
+      // D = c0 + c1 s (key_dot; the key prepared for fixed_mul), at input i's
       // slot for this limb: the position of l among dot.mask's limbs
       const uint32_t kd = (uint32_t)__builtin_popcount(dot.mask & ((1u << l) - 1));
       const uint32_t nd = (uint32_t)__builtin_popcount(dot.mask);

@@ -129,7 +129,8 @@ __global__ void k_sub_product(const uint64_t* __restrict__ x, const uint64_t* __
 
 // D = c0 + c1 s on limbs 0..nl-1 of count ciphertexts at cts + i ct_stride
 // ([c0 | c1], L limbs each), with the secret key prepared (k_to_montgomery): the
-// decryption's c0 + c1 s (ciphertext.rs:332-341), lazily in [0, 3q). For a
+// decryption's c0 + c1 s (ciphertext.rs:332-341), in [0, 3q), on pm limbs
+// folded below 1.1q. For a
 // product ciphertext (c0 pt, c1 pt) the decryption is pt (c0 + c1 s), so one
 // D per input serves every plaintext it is multiplied by.
 __global__ void k_key_dot(const uint64_t* __restrict__ cts, uint64_t ct_stride, const uint64_t* __restrict__ skm,

@@ -277,7 +277,7 @@ struct th_ctx {
 struct th_sk {
   th_ctx* ctx;
   uint64_t* d;                     // L x N, NTT domain
-  mutable uint64_t* dm = nullptr;  // the same in Montgomery form (launch_to_montgomery), made on first use
+  mutable uint64_t* dm = nullptr;  // the same prepared (launch_to_montgomery), made on first use
 };
 struct th_pk {
   th_ctx* ctx;
@@ -305,7 +305,7 @@ struct th_lora {
   uint64_t n_deltas = 0;
   std::vector<void*> owned;
   uint64_t* pts = nullptr;     // n_batches x L x N, NTT domain
-  uint64_t* ptm = nullptr;     // the same in Montgomery form (launch_to_montgomery)
+  uint64_t* ptm = nullptr;     // the same prepared (launch_to_montgomery)
   double* hidden = nullptr;    // n_in x d
   uint8_t* u = nullptr;        // n_in x N
   int64_t *e0 = nullptr, *e1 = nullptr;

@@ -133,7 +133,7 @@ const uint64_t* pk_pairs(th_ctx* c, const th_pk* pk) {
   return pk->dp;
 }
 
-// The secret key in Montgomery form, made likewise.
+// The secret key prepared (Montgomery form, unchanged on pm limbs), made likewise.
 const uint64_t* sk_montgomery(th_ctx* c, const th_sk* sk) {
   if (!sk->dm) {
     uint64_t* p = (uint64_t*)c->pool.get((size_t)c->L * c->N * 8);

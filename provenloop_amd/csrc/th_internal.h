@@ -90,7 +90,7 @@ struct NttArgs {
   const uint64_t* key;        // secret key, L x N (DOT)
   const double* segw;         // segment weight pairs, N x 2 (SEGSUM)
   uint32_t cols;              // segments per job (SEGSUM)
-  uint32_t stream;            // forward split passes: nontemporal hints (set by the launchers)
+  uint32_t pad_;
 };
 
 // One product ct x pt of a LoRA set, rescaled and decrypted on limb 0 into
@@ -99,8 +99,8 @@ struct NttArgs {
 struct RescaleDecryptJob {
   const uint64_t* y;
   const uint64_t* x;
-  const uint64_t* d;    // c0 + c1 s of the product's input on limb 0, in [0, 3q) (k_key_dot)
-  const uint64_t* ptm;  // the plaintext's limb 0 in Montgomery form
+  const uint64_t* d;    // c0 + c1 s of the product's input on limb 0 (k_key_dot)
+  const uint64_t* ptm;  // the plaintext's limb 0, prepared (launch_to_montgomery)
   double* seg;          // cols segment sums
   double scale;         // the rescaled ciphertext's scale
 };
@@ -108,7 +108,7 @@ struct RescaleDecryptArgs {
   LimbTable lc;                 // limb 0 is lc[0]
   const BarrettConst* bc;       // limb 0
   const RescaleConst* rc;       // limb 0 at the products' level
-  const uint64_t* skm;          // the secret key's limb 0 in Montgomery form
+  const uint64_t* skm;          // the secret key's limb 0, prepared
   const double* segw;           // segment weight pairs, N x 2 (NTT_STORE_SEGSUM)
   const RescaleDecryptJob* jobs;
   uint32_t cols;                // segments per job, at most NTT_SEGSUM_FUSED_MAX_COLS
@@ -143,10 +143,10 @@ hipError_t allow_full_lds() {
 
 // Launch njobs forward (inverse=false) or inverse negacyclic NTTs of size 2^logn.
 hipError_t launch_ntt(int logn, bool inverse, const NttArgs& a, uint32_t njobs, hipStream_t s);
-// The decryption's D = c0 + c1 s (in [0, 3q)), formed by the encrypt row
-// passes on the limbs in mask instead of storing c0 and c1 there: input i's D
-// on the k-th limb of mask at out + (i n + k) N for n limbs in mask; skm =
-// the secret key (L x N) in Montgomery form.
+// The decryption's D = c0 + c1 s (in [0, 3q), on pm limbs below 1.1q), formed
+// by the encrypt row passes on the limbs in mask instead of storing c0 and c1
+// there: input i's D on the k-th limb of mask at out + (i n + k) N for n limbs
+// in mask; skm = the secret key (L x N), prepared (launch_to_montgomery).
 struct EncDot {
   uint32_t mask;
   const uint64_t* skm;
@@ -180,7 +180,7 @@ hipError_t launch_rescale(int logn, const NttArgs& inv, uint32_t ninv, const Ntt
 hipError_t launch_rescale_decrypt(int logn, const RescaleDecryptArgs& a, uint32_t njobs, hipStream_t s);
 // The same for nb batches on the split kernels (N = 8192 .. 32768), from the
 // products' last limbs: inv = the 2 nb inverse jobs (X, Y of batch b at 2b,
-// 2b+1; src = ct's last limb, aux = pt's last limb in Montgomery form, load
+// 2b+1; src = ct's last limb, aux = pt's last limb, prepared, load
 // NTT_LOAD_MULM, dst = the batch's x, y work areas); partials: scratch of
 // nb x cols x N/16 doubles. The segment sums equal launch_rescale_decrypt's
 // bit for bit at N = 16384.
@@ -188,8 +188,8 @@ hipError_t launch_rescale_decrypt_split(int logn, const NttArgs& inv, const Resc
                                         double* partials, hipStream_t s);
 // A plain batched decryption with segment sums on the split kernels (N =
 // 8192 .. 32768) for nb batches: row = the nb inverse jobs of c0 + c1 s on
-// limb 0 (src = c0, aux = c1, load NTT_LOAD_DOTM with row.key the secret key
-// in Montgomery form, dst = the batch's work area, which a.jobs[b].y names
+// limb 0 (src = c0, aux = c1, load NTT_LOAD_DOTM with row.key the secret key,
+// prepared, dst = the batch's work area, which a.jobs[b].y names
 // too); a.jobs[b].seg and .scale as for the rescale-decrypt; partials: nb x
 // cols x N/16 doubles. At N = 16384 the sums equal, bit for bit, those of the
 // whole-polynomial decrypt's segment-sum epilogue (NTT_STORE_SEGSUM).
