@@ -543,21 +543,25 @@ __device__ __forceinline__ uint32_t column_part(uint32_t p) {
 }
 
 // Wavefronts per SIMD of a split kernel, or `any`. The plain inverse passes on
-// pm limbs need 92 to 94 registers, which allows five, but their LDS holds 18
+// pm limbs need 92 registers, which allows five, but their LDS holds 18
 // workgroups on a CU, so SIMDs hold four or five, in rounds that do not end
-// together: 16 on a CU through the LDS size change nothing, four on each SIMD
-// do, and in the column pass, whose wavefronts each store 16 lines of the
-// natural layout, three. A pass of 64 transforms of 4 limbs at N = 32768 with
-// the copy before it: 75.4 us with neither, 73.0 with four in both, 71.4 with
-// three in the column pass, 73.5 with three in the row pass; 256 of them 334,
-// 326, 319, 335; N = 16384, 256: 174, 168, 161, 169. In place on data the
-// caches hold the passes stay within 2 %. IntArith's take 99 registers and more,
-// four wavefronts, by themselves.
+// together. Where the data outgrow the caches (STREAM, inverse_stream) four on
+// each SIMD are faster (16 on a CU through the LDS size change nothing), and in
+// the column pass, whose wavefronts each store 16 lines of the natural layout,
+// three. 64 transforms of 4 limbs at N = 32768 (64 MiB) with the copy before
+// them: 75.4 us without, 73.0 with four in both, 71.4 with three in the column
+// pass, 73.5 with three in the row pass; 256 of them 334, 326, 319, 335; N =
+// 16384, 256: 174, 168, 161, 169. Below 64 MiB passes behind a copy gain 2 % at
+// most, and passes in place on cached data lose 3 to 5 % (33 to 52 MB).
+// IntArith's passes take 99 registers and more, four wavefronts, by themselves.
 constexpr int MAX_WAVES = 8;
-template <class BIG, bool INV, bool COLUMN, uint32_t LD, uint32_t ST>
+template <bool INV, bool COLUMN, bool STREAM>
 constexpr int split_waves(int any) {
-  if (!std::is_same_v<BIG, PmArith> || !INV || LD != NTT_LOAD_NONE || ST != NTT_STORE_NONE) return any;
-  return COLUMN ? 3 : 4;
+  return INV && STREAM ? (COLUMN ? 3 : 4) : any;
+}
+template <int LOGN>
+static bool inverse_stream(uint32_t njobs) {
+  return ((uint64_t)njobs * 8 << LOGN) >= (64u << 20);
 }
 
 // Workgroup b works on part b % PARTS of job b / PARTS. The pass that reads
@@ -566,7 +570,7 @@ constexpr int split_waves(int any) {
 // destination only.
 template <class BIG, int LOGN, bool INV, bool COLUMN, uint32_t LD, uint32_t ST, bool STREAM = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
-    split_waves<BIG, INV, COLUMN, LD, ST>(1), split_waves<BIG, INV, COLUMN, LD, ST>(MAX_WAVES)))) void
+    split_waves<INV, COLUMN, STREAM>(1), split_waves<INV, COLUMN, STREAM>(MAX_WAVES)))) void
 ntt_split_kernel(NttArgs a) {
   using S = Split<LOGN>;
   // the forward row pass with a fused rescale store, and the inverse row pass
@@ -883,6 +887,15 @@ static hipError_t launch_split_t(const NttArgs& a, uint32_t njobs, hipStream_t s
                            hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, false, false, NTT_LOAD_NONE, ST>), grid, block,
                                               0, s, a);
                          } else {
+                           if constexpr (std::is_same_v<BIG, PmArith> && LD == NTT_LOAD_NONE) {
+                             if (inverse_stream<LOGN>(njobs)) {
+                               hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, false, LD, NTT_STORE_NONE, true>),
+                                                  grid, block, 0, s, a);
+                               hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, true, LD, NTT_STORE_NONE, true>),
+                                                  grid, block, 0, s, a);
+                               return hipGetLastError();
+                             }
+                           }
                            hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, false, LD, NTT_STORE_NONE>), grid, block,
                                               0, s, a);
                            hipLaunchKernelGGL((ntt_split_kernel<BIG, LOGN, true, true, NTT_LOAD_NONE, NTT_STORE_NONE>), grid,

@@ -85,3 +85,17 @@ def test_ciphertext_operations(kind):
     for got, exp in ((ct, rct), (prod, rprod), (res, rres)):
         assert all(np.array_equal(a, b) for a, b in zip(eng.ct_download(got), ref.ct_data(exp)))
         assert np.array_equal(eng.decrypt(got, sk), ref.decrypt(exp, rsk))
+
+
+@pytest.mark.parametrize("n,polys", [(8192, 341), (8192, 342), (16384, 171), (32768, 85), (32768, 86)])
+def test_inverse_batches_around_64_mib(n, polys):
+    """Larger batches take instances of their own from 64 MiB of residues on (3 limbs each)."""
+    q = _chain("pm", n)
+    ctx = tensafe_he.CkksContext(n, moduli=q)
+    rng = np.random.default_rng(polys)
+    x = np.stack([rng.integers(0, m, (polys, n), dtype=np.uint64) for m in q], axis=1)
+    x[0] = x[-1] = np.array(q, np.uint64)[:, None] - np.uint64(1)
+    inv = ctx.ntt_inverse(x)
+    for p in (0, polys // 2, polys - 2, polys - 1):
+        for l, m in enumerate(q):
+            assert np.array_equal(inv[p, l], orc.ntt_inverse(x[p:p + 1, l], m)[0]), (p, l)

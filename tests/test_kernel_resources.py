@@ -74,11 +74,13 @@ def _find(kernels, pattern):
 
 
 @pytest.mark.parametrize("logn", [13, 14, 15])
-def test_plain_inverse_passes_keep_their_wavefronts(kernels, logn):
-    """Row pass four wavefronts per SIMD, column pass three, on chains of folded primes."""
+def test_large_inverse_passes_keep_their_wavefronts(kernels, logn):
+    """On chains of folded primes, launches larger than the caches: row pass four wavefronts per SIMD, column pass
+    three; the smaller ones' instances as many as their registers allow."""
     for column, waves in ((0, 4), (1, 3)):
-        name = f"16ntt_split_kernelI{PM}Li{logn}ELb1ELb{column}ELj0ELj0ELb0E"
-        assert [w for w, _ in _find(kernels, name).values()] == [waves]
+        name = f"16ntt_split_kernelI{PM}Li{logn}ELb1ELb{column}ELj0ELj0ELb"
+        assert [w for w, _ in _find(kernels, name + "1E").values()] == [waves]
+        assert [w for w, _ in _find(kernels, name + "0E").values()] == [5]
 
 
 def test_split_kernels_do_not_spill(kernels):
