@@ -353,9 +353,10 @@ int th_pk_import(th_ctx* ctx, const uint8_t* buf, size_t len, th_pk** out);
 
 /* ---------------------------------------------------------------- raw transforms */
 /* In-place forward / inverse negacyclic NTT (ntt.rs:79-141) of `count`
- * polynomials, each `limbs` consecutive limb-polynomials of N u64 using
- * moduli q_0 .. q_{limbs-1}. `polys` is a host pointer (on_device == 0) or a
- * device pointer (on_device == 1; asynchronous on the context stream). */
+ * polynomials, each `limbs` consecutive limb-polynomials of N u64 residues
+ * (limb l's in [0, q_l)) for moduli q_0 .. q_{limbs-1}. `polys` is a host
+ * pointer (on_device == 0) or a device pointer (on_device == 1; asynchronous
+ * on the context stream). */
 int th_ntt_forward_batch(th_ctx* ctx, uint64_t* polys, size_t count, uint32_t limbs, int on_device);
 int th_ntt_inverse_batch(th_ctx* ctx, uint64_t* polys, size_t count, uint32_t limbs, int on_device);
 /* Device-memory helpers for callers without their own allocator. th_dev_free
