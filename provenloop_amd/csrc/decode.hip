@@ -282,7 +282,7 @@ hipError_t launch_decode(const DecodeJob* jobs, uint32_t njobs, const DecodeCons
   if (!njobs) return hipSuccess;
   if (cols == 0) {  // slots only
     const uint32_t lp = decode_parts_log(logn, njobs), M = (1u << logn) >> lp;
-    const uint32_t threads = M / 8 < 64 ? 64 : (M / 8 > DEC_THREADS ? DEC_THREADS : M / 8);
+    const uint32_t threads = decode_threads(logn, lp, njobs);
     const uint32_t fin = lp >= 2 ? M << (lp - 2) : M;
     const size_t lds = fft_part_lds(logn, lp);
 #define TH_SLOTS(LP)                                                                                             \

@@ -19,7 +19,7 @@ constexpr bool poll_download(size_t bytes) { return bytes > (16u << 10) && bytes
 
 // A transform of N complex values (encoder, decoder) is cut into 2^lp parts of
 // N / 2^lp values, one workgroup each, of an eighth as many threads (64 to
-// 1024); the result is the same for any split. From 8 parts on a part stages
+// 1024; decodes: decode_threads); the result is the same for any split. From 8 parts on a part stages
 // its twiddles in LDS beside its values (fft_part_lds): 4096 values take 72
 // KiB, 136 with the twiddles, so at N = 32768 a CU holds one workgroup of 512
 // threads; 8192 values take 144 KiB with 1024 threads.
@@ -49,6 +49,23 @@ constexpr uint32_t decode_parts_log(uint32_t logn, uint32_t njobs) {
   uint32_t lp = logn <= 12 ? 0 : logn == 13 ? 1 : 2;
   while (lp < 4 && logn - lp > 10 && ((uint64_t)njobs << (lp + 1)) <= DECODE_FILL) ++lp;
   return lp;
+}
+
+// Threads of a decode's part. A thread converts its residues one after another
+// (through 128 bits on the CRT path), so a quarter as many threads as values
+// where they find room: in parts of up to 2048 values, and in larger ones while
+// a CU has only one of them and no staged twiddles. An eighth / a quarter, CRT:
+//   N = 1024, 256 decodes     74.4 / 70.7 us    N = 2048, 256   84.1 / 82.4
+//   N = 16384, one            48.6 / 46.4       N = 16384, 64   85.0 / 82.8
+//   N = 4096, 255             96.0 / 93.8       N = 8192, 64    66.2 / 64.2
+// and where two parts share a CU or twiddles are staged:
+//   N = 8192, 256            128.6 / 137.8      N = 16384, 128  112.3 / 122.6
+//   N = 32768, 24 (limb 0)    62.7 / 64.5
+constexpr uint32_t decode_threads(uint32_t logn, uint32_t lp, uint32_t njobs) {
+  const uint32_t M = (1u << logn) >> lp;
+  const bool room = M <= 2048 || (lp < 3 && ((uint64_t)njobs << lp) <= DECODE_FILL);
+  const uint32_t t = room ? M / 4 : M / 8;
+  return t < 64 ? 64 : t > 1024 ? 1024 : t;
 }
 
 // Places for short job lists in a ring of `cap` bytes, handed out in turn on

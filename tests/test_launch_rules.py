@@ -49,6 +49,17 @@ def test_decodes_are_cut_into_at_most_one_part_per_cu(evaluate):
     assert [got[15, j] for j in (16, 17, 32, 33, 64, 256)] == [4, 3, 3, 2, 2, 2]
 
 
+def test_decode_threads(evaluate):
+    """At most 8 values a thread (dit_stages_reg), at most 1024 threads, a quarter of the values where a CU has room."""
+    cases = [(logn, jobs) for logn in range(10, 16) for jobs in (1, 16, 17, 33, 64, 65, 128, 129, 256, 257, 5000)]
+    lps = evaluate([f"th::decode_parts_log({n}, {j})" for n, j in cases])
+    threads = evaluate([f"th::decode_threads({n}, th::decode_parts_log({n}, {j}), {j})" for n, j in cases])
+    for (logn, jobs), lp, t in zip(cases, lps, threads):
+        m = 1 << logn >> lp
+        assert 64 <= t <= 1024 and t % 64 == 0 and m <= 8 * t
+        assert (t == min(1024, m // 4)) == (m <= 2048 or m == 8192 or (lp < 3 and jobs << lp <= 256))
+
+
 def test_encodes_fill_two_workgroups_per_cu(evaluate):
     cases = [(13, 1), (13, 64), (13, 255), (13, 256), (14, 28), (14, 64), (14, 128), (14, 672), (15, 28), (15, 64), (10, 1)]
     assert evaluate([f"th::encode_parts_log({n}, {j})" for n, j in cases]) == [3, 3, 2, 1, 4, 3, 2, 2, 4, 3, 0]
