@@ -624,10 +624,10 @@ ntt_split_kernel(NttArgs a) {
 // the launch takes one inverse and one forward pass instead of the inverse
 // and nf forward passes in turn.
 // Wavefronts per SIMD: three. With Shoup products that needs the arithmetics'
-// code kept apart (with_arith) at N <= 16384 (160 to 164 registers, against 183
-// to 190 and two wavefronts, or 16 registers spilled at three: 200 products
-// 282 us against 291 and 296), and spills all the same at N = 32768, which has
-// two (64 products on 8 limbs: 276 us, 293 at three).
+// code kept apart (with_arith) at N <= 16384: 160 to 164 registers, against 183
+// to 190 and two wavefronts, or three and 16 registers spilled (token at N =
+// 16384 on such a chain: 385 us against 396 and 399). At N = 32768 it spills all
+// the same, so two there (64 products on 8 limbs: 276 us, 293 at three).
 template <class BIG, int LOGN>
 constexpr bool RESCALE_APART = std::is_same_v<BIG, IntArith> && LOGN < 15;
 template <class BIG, int LOGN, bool STREAM>
